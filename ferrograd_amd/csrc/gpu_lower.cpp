@@ -1014,31 +1014,275 @@ std::vector<UOp> loads_in(const UOp& v) {
   return out;
 }
 
+// The reduced value and its ranges (outermost first) with every pair of
+// adjacent ranges that all loads walk as one (the outer one's stride is the
+// inner one's extent times its stride) merged: a sum over both axes of a
+// [5000, 3001] tensor has one range of 15,005,000.
+struct RowTerms {
+  UOp value;
+  std::vector<UOp> ranges;
+  int64_t terms = 1;
+};
+
+RowTerms row_terms(const KernelInfo& ki) {
+  const UOp& R = ki.reduces[0];
+  RowTerms t{R.src(0), std::vector<UOp>(R.srcs().begin() + 1, R.srcs().end()), 1};
+  for (auto& r : t.ranges) t.terms *= range_extent(r);
+  // Term numbers are int32; an empty reduction has none.
+  if (t.terms == 0 || t.terms >= (int64_t(1) << 31) - (int64_t(1) << 20)) return t;
+  // Ranges are merged only where nothing but load indexes uses them.
+  UOpSet seen;
+  bool only_indexes = true;
+  std::function<void(const UOp&)> walk = [&](const UOp& n) {
+    if (!seen.insert(n).second || n.op() == Op::Load) return;
+    if (n.op() == Op::Range)
+      for (auto& r : t.ranges) only_indexes = only_indexes && r != n;
+    for (auto& x : n.srcs()) walk(x);
+  };
+  walk(t.value);
+  if (!only_indexes) return t;
+  int64_t next = 0;
+  for (auto& n : t.value.toposort())
+    if (n.op() == Op::Range) next = std::max(next, n.arg().a + 1);
+  for (auto& r : ki.out_ranges) next = std::max(next, r.arg().a + 1);
+  for (size_t i = t.ranges.size(); i-- > 1;) {
+    const UOp outer = t.ranges[i - 1], inner = t.ranges[i];
+    const int64_t ei = range_extent(inner);
+    bool one = true;
+    for (auto& ld : loads_in(t.value)) {
+      const Affine a = affine_of(ld.src(0).src(1));
+      one = one && a.ok && a.coef(outer) == ei * a.coef(inner);
+    }
+    if (!one) continue;
+    const UOp n = UOp::const_int(range_extent(outer) * ei, DType::I32(), inner.device());
+    const UOp zero = UOp::const_int(0, DType::I32(), inner.device());
+    const UOp merged = UOp::make_new(Op::Range, inner.dtype(), {n}, Arg::range(next++, inner.arg().range_kind()));
+    t.value = substitute_with_map(t.value, {{outer, zero}, {inner, merged}});
+    t.ranges.erase(t.ranges.begin() + static_cast<std::ptrdiff_t>(i));
+    t.ranges[i - 1] = merged;
+  }
+  return t;
+}
+
+// Whether every load that moves along `r_in` is unit-stride and 16-byte
+// aligned in steps of 4 terms.
+bool row_loads_vec4(const UOp& value, const UOp& r_in) {
+  for (auto& ld : loads_in(value)) {
+    Affine a = affine_of(ld.src(0).src(1));
+    int64_t c = a.ok ? a.coef(r_in) : -1;
+    if (c == 0) continue;
+    if (!a.ok || c != 1 || a.c0 % 4 != 0 || (ld.dtype().kind != DTypeKind::F32 && ld.dtype().kind != DTypeKind::I32))
+      return false;
+    for (auto& t : a.terms)
+      if (t.first != r_in && t.second % 4 != 0) return false;
+  }
+  return true;
+}
+
+// ── RowReduce over few outputs: split over workgroups ──────────────────────
+// One workgroup per output (render_row_reduce's largest group) leaves the chip
+// idle when there are few outputs of many terms: the sum of a whole
+// [5000, 3001] tensor ran on one workgroup in 7,886 us, 64 rows of 2^18 terms
+// in 23.6 us and nine rows of 1,864,135 in 597 us. Here the terms of each
+// output are cut into chunks, one workgroup each (`<name>_part`, one partial
+// per chunk in program-owned scratch, [output][chunk]); `<name>_fin` folds an
+// output's partials in chunk order with one workgroup and runs the epilogue.
+// Fixed order, no atomics. Same box, part and fin together: 7,886 -> 14.4 us,
+// 23.6 -> 12.6 us, 597 -> 15.0 us; at those sizes bound by HBM and the
+// Infinity Cache (10.4 us for the first's 60 MB), below a few MiB by its two
+// launches.
+//
+// From 512 outputs on the unsplit kernel has two workgroups per CU (513 rows
+// of 32,704 run at 6.3 TB/s). Below, the split pays from about 64 steps of an
+// unsplit thread, whose loads then take as long as the second launch: nine
+// rows of 116,508 (114 steps) 8.7 us unsplit, 8.0 us split; rows of 7,281 (28
+// steps) 4.6 us unsplit.
+constexpr int64_t kRowSplitMaxOutputs = 512;
+constexpr int64_t kRowSplitMinSteps = 64;
+constexpr int64_t kRowSplitWorkgroups = 2048;  // eight 256-thread workgroups per CU
+constexpr int64_t kRowSplitChunkSteps = 8;     // fewest steps of a chunk's threads
+
+struct RowSplit {
+  UOp value;
+  std::vector<UOp> ranges;
+  int V = 1;                    // terms per step along the innermost range
+  int64_t groups = 0;           // steps of V terms, over all threads
+  int64_t tail = 0;             // terms past the last whole step (one range, one output)
+  int64_t chunks = 0, per = 0;  // workgroups per output, groups per chunk
+};
+
+// `steps`: the steps a thread of the unsplit kernel runs.
+bool row_split(const KernelInfo& ki, const RowTerms& rt, int64_t steps, RowSplit* sp) {
+  const int64_t nout = total_outputs(ki);
+  if (nout >= kRowSplitMaxOutputs || steps < kRowSplitMinSteps) return false;
+  if (rt.terms >= (int64_t(1) << 31) - (int64_t(1) << 20)) return false;
+  for (auto& ld : loads_in(rt.value))
+    if (!affine_of(ld.src(0).src(1)).ok) return false;
+  sp->value = rt.value;
+  sp->ranges = rt.ranges;
+  const int64_t L = range_extent(rt.ranges.back());
+  // The one range of one output may end in a partial step.
+  const bool whole = L % 4 == 0 || (rt.ranges.size() == 1 && nout == 1 && L >= 4);
+  sp->V = whole && row_loads_vec4(rt.value, rt.ranges.back()) ? 4 : 1;
+  sp->groups = rt.terms / sp->V;
+  sp->tail = rt.terms % sp->V;
+  const int64_t rounds = (sp->groups + 255) / 256;  // of one workgroup
+  const int64_t want = kRowSplitWorkgroups / nout;
+  sp->per = 256 * std::max<int64_t>(kRowSplitChunkSteps, (rounds + want - 1) / want);
+  sp->chunks = (sp->groups + sp->per - 1) / sp->per;
+  return true;
+}
+
+RenderedKernel render_row_reduce_split(const KernelInfo& ki, const RowSplit& sp, const std::string& name) {
+  const UOp& R = ki.reduces[0];
+  const Op rop = R.arg().rop;
+  const DType dt = R.dtype();
+  const std::string ct = ctype(dt), init = init_lit(rop, dt);
+  const int64_t nout = total_outputs(ki);
+  const UOp r_in = sp.ranges.back();
+  auto str = [](int64_t v) { return std::to_string(v); };
+  auto sig = [&](const std::string& fn) {
+    std::string s = signature(ki, fn, 256);
+    return s.substr(0, s.size() - 1) + ", " + ct + "* __restrict__ fg_scratch)";
+  };
+  // The total over the workgroup, in every thread of its first wave.
+  auto fold_workgroup = [&](Emitter& em, const std::string& acc) {
+    std::istringstream is(wave_reduce(acc, 64, rop, dt));
+    for (std::string l; std::getline(is, l);) em.line(l);
+    em.line("__shared__ " + ct + " fg_part[4];");
+    em.line("if ((tid & 63) == 0) fg_part[tid >> 6] = " + acc + ";");
+    em.line("__syncthreads();");
+    em.line(acc + " = " + combine(rop, combine(rop, combine(rop, "fg_part[0]", "fg_part[1]"), "fg_part[2]"), "fg_part[3]") +
+            ";");
+  };
+
+  Emitter p1;
+  p1.set_nontemporal_loads(true);
+  p1.set_streaming_ranges(ki.out_ranges);
+  p1.line("const int tid = threadIdx.x;");
+  p1.line("const int chunk = (int)(blockIdx.x % " + str(sp.chunks) + ");");
+  p1.line("const long ob = blockIdx.x / " + str(sp.chunks) + ";");
+  decode_outputs(p1, ki, "ob", UOp());
+  p1.line("const int g0 = chunk * " + str(sp.per) + ";");
+  p1.line("const int gn = " + str(sp.groups) + " - g0 < " + str(sp.per) + " ? " + str(sp.groups) + " - g0 : " + str(sp.per) +
+          ";");
+  p1.line(ct + " racc = " + init + ";");
+  // The term (step `g`, its first of V) as the ranges' indexes.
+  auto decode = [&](const std::string& g) {
+    std::string rest = g;
+    for (size_t i = sp.ranges.size(); i-- > 0;) {
+      const bool in = i + 1 == sp.ranges.size();
+      const int64_t e = range_extent(sp.ranges[i]) / (in ? sp.V : 1);
+      const std::string v = "rt" + str(static_cast<int64_t>(i));
+      const std::string mul = in && sp.V > 1 ? " * " + str(sp.V) : "";
+      if (i == 0) {
+        p1.line("const int " + v + " = " + rest + mul + ";");
+      } else {
+        p1.line("const int " + v + " = (" + rest + " % " + str(e) + ")" + mul + ";");
+        p1.line("const int " + v + "q = " + rest + " / " + str(e) + ";");
+        rest = v + "q";
+      }
+      p1.define_range(sp.ranges[i], v);
+    }
+  };
+  auto fold = [&](int V) {
+    std::string group;
+    if (V == 4) {
+      p1.set_lane_range(r_in, 4);
+      std::vector<std::string> l;
+      for (int u = 0; u < 4; u++) l.push_back(p1.val(sp.value, u));
+      group = combine(rop, combine(rop, combine(rop, l[0], l[1]), l[2]), l[3]);
+    } else {
+      group = p1.val(sp.value, 0);
+    }
+    p1.line("racc = " + combine(rop, "racc", group) + ";");
+    p1.clear_lane_range();
+  };
+  p1.line("const int gfull = gn / 256;");
+  p1.open_scope("#pragma unroll 8\nfor (int it = 0; it < gfull; it++) {", "}");
+  p1.line("const int g = g0 + it * 256 + tid;");
+  decode("g");
+  fold(sp.V);
+  p1.close_scope();
+  p1.open_scope("if (tid < gn - gfull * 256) {", "}");
+  p1.line("const int g = g0 + gfull * 256 + tid;");
+  decode("g");
+  fold(sp.V);
+  p1.close_scope();
+  if (sp.tail) {
+    p1.open_scope("if (chunk == " + str(sp.chunks - 1) + " && tid < " + str(sp.tail) + ") {", "}");
+    p1.line("const int rt0 = " + str(sp.groups * sp.V) + " + tid;");
+    p1.define_range(r_in, "rt0");
+    fold(1);
+    p1.close_scope();
+  }
+  RenderedKernel rk;
+  rk.name = name;
+  rk.kind = kernel_class_name(KernelClass::RowReduce);
+  rk.block[0] = 256;
+  rk.grid[0] = static_cast<unsigned>(nout * sp.chunks);
+  if (sp.chunks == 1) {  // a short reduction whose innermost range was shorter still: one pass
+    p1.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
+      FG_CHECK(RR == R, "row reduce renders exactly one reduction");
+      fold_workgroup(p1, "racc");
+      p1.remember_here(RR, lane, "racc");
+      return "racc";
+    };
+    const std::string v = p1.val(ki.value, 0);
+    p1.line("if (tid == 0) " + pname(ki.out_param) + "[" + p1.idx(ki.out_index, 0) + "] = " + v + ";");
+    rk.source = std::string(kPrelude) + signature(ki, name, 256) + " {\n" + p1.code() + "}\n";
+    return rk;
+  }
+  fold_workgroup(p1, "racc");
+  p1.line("if (tid == 0) fg_scratch[blockIdx.x] = racc;");
+
+  Emitter p2;
+  p2.line("const int tid = threadIdx.x;");
+  p2.line("const long ob = blockIdx.x;");
+  decode_outputs(p2, ki, "ob", UOp());
+  p2.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
+    FG_CHECK(RR == R, "row reduce renders exactly one reduction");
+    p2.line(ct + " racc = " + init + ";");
+    p2.line("#pragma unroll 8");
+    p2.line("for (int c = tid; c < " + str(sp.chunks) + "; c += 256) racc = " +
+            combine(rop, "racc", "fg_scratch[ob * " + str(sp.chunks) + " + c]") + ";");
+    fold_workgroup(p2, "racc");
+    p2.remember_here(RR, lane, "racc");
+    return "racc";
+  };
+  const std::string v = p2.val(ki.value, 0);
+  p2.line("if (tid == 0) " + pname(ki.out_param) + "[" + p2.idx(ki.out_index, 0) + "] = " + v + ";");
+
+  rk.source = std::string(kPrelude) + sig(name + "_part") + " {\n" + p1.code() + "}\n" + sig(name + "_fin") + " {\n" +
+              p2.code() + "}\n";
+  LaunchSpec a, b;
+  a.func = name + "_part";
+  a.grid[0] = rk.grid[0];
+  a.block[0] = 256;
+  b.func = name + "_fin";
+  b.grid[0] = static_cast<unsigned>(nout);
+  b.block[0] = 256;
+  rk.launches = {a, b};
+  rk.scratch_bytes = static_cast<size_t>(nout * sp.chunks) * dt.size_bytes();
+  return rk;
+}
+
 // ── RowReduce ───────────────────────────────────────────────────────────────
 RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) {
   const UOp& R = ki.reduces[0];
   Op rop = R.arg().rop;
   DType dt = R.dtype();
-  std::vector<UOp> ranges(R.srcs().begin() + 1, R.srcs().end());
+  const RowTerms rt = row_terms(ki);
+  const std::vector<UOp>& ranges = rt.ranges;
   const UOp r_in = ranges.back();
   int64_t L = range_extent(r_in);
   int T = std::min<int>(256, pow2_floor(std::max<int64_t>(1, L / 16)));
   int OPW = 256 / T;  // outputs per workgroup
   int64_t NOUT = total_outputs(ki);
   // Vector width along r_in: all lane-dependent loads unit-stride and aligned.
-  int V = (L % 4 == 0) ? 4 : 1;
-  if (V == 4) {
-    for (auto& ld : loads_in(R.src(0))) {
-      Affine a = affine_of(ld.src(0).src(1));
-      int64_t c = a.ok ? a.coef(r_in) : -1;
-      if (c == 0) continue;
-      bool ok = a.ok && c == 1 && a.c0 % 4 == 0 &&
-                (ld.dtype().kind == DTypeKind::F32 || ld.dtype().kind == DTypeKind::I32);
-      for (auto& t : a.terms)
-        if (t.first != r_in && t.second % 4 != 0) ok = false;
-      if (!ok) V = 1;
-    }
-  }
+  const int V = L % 4 == 0 && row_loads_vec4(rt.value, r_in) ? 4 : 1;
+  RowSplit sp;
+  if (L > 0 && row_split(ki, rt, rt.terms / L * ((L + T * V - 1) / (T * V)), &sp)) return render_row_reduce_split(ki, sp, name);
   Emitter em;
   em.set_nontemporal_loads(true);
   em.set_streaming_ranges(ki.out_ranges);
@@ -1049,7 +1293,7 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   // read by several outputs: the same row for every output column of a
   // narrow matmul.
   bool shared_rows = false;
-  for (auto& ld : loads_in(R.src(0))) {
+  for (auto& ld : loads_in(rt.value)) {
     const UOp& ix = ld.src(0).src(1);
     if (!em.depends_on(ix, r_in.get())) continue;
     for (auto& o : ki.out_ranges)
@@ -1091,10 +1335,10 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
       if (V == 4) {
         em.set_lane_range(r_in, 4);
         std::vector<std::string> lanes;
-        for (int u = 0; u < 4; u++) lanes.push_back(em.val(R.src(0), u));
+        for (int u = 0; u < 4; u++) lanes.push_back(em.val(rt.value, u));
         group = combine(rop, combine(rop, combine(rop, lanes[0], lanes[1]), lanes[2]), lanes[3]);
       } else {
-        group = em.val(R.src(0), 0);
+        group = em.val(rt.value, 0);
       }
       em.line(acc + " = " + combine(rop, acc, group) + ";");
       if (V == 4) em.clear_lane_range();
