@@ -688,19 +688,20 @@ int pow2_floor(int64_t x) {
 }
 
 // Decode the flattened output index `lin` into range variables (innermost
-// range varies fastest). Emits `int idxN = ...;` lines, skipping `skip`.
-void decode_outputs(Emitter& em, const KernelInfo& ki, const std::string& lin, const UOp& skip) {
+// range varies fastest). Emits `int idxN = ...;` lines, skipping `skipped`.
+void decode_outputs(Emitter& em, const KernelInfo& ki, const std::string& lin, const std::vector<UOp>& skipped) {
+  auto skip = [&](const UOp& r) { return std::find(skipped.begin(), skipped.end(), r) != skipped.end(); };
   std::string rest = lin;
   bool first = true;
   for (size_t i = ki.out_ranges.size(); i-- > 0;) {
     const UOp& r = ki.out_ranges[i];
-    if (r == skip) continue;
+    if (skip(r)) continue;
     std::string name = "idx" + std::to_string(r.arg().a);
     int64_t e = ki.out_ext[i];
     // Is this the outermost remaining range? Then no modulo is needed.
     bool outermost = true;
     for (size_t j = 0; j < i; j++)
-      if (ki.out_ranges[j] != skip) outermost = false;
+      if (!skip(ki.out_ranges[j])) outermost = false;
     if (outermost) em.line("const int " + name + " = (int)(" + rest + ");");
     else em.line("const int " + name + " = (int)((" + rest + ") % " + std::to_string(e) + ");");
     em.define_range(r, name);
@@ -712,6 +713,10 @@ void decode_outputs(Emitter& em, const KernelInfo& ki, const std::string& lin, c
     first = false;
   }
   (void)first;
+}
+
+void decode_outputs(Emitter& em, const KernelInfo& ki, const std::string& lin, const UOp& skip) {
+  decode_outputs(em, ki, lin, std::vector<UOp>{skip});
 }
 
 UOp pick_fast_output(const KernelInfo& ki) {
@@ -1415,6 +1420,31 @@ RenderedKernel render_row_reduce_split(const KernelInfo& ki, const RowSplit& sp,
   return rk;
 }
 
+// ── RowReduce read by a whole row of outputs ───────────────────────────────
+// A kernel whose reduction does not move with some output ranges (a softmax
+// gradient's row sum inside an elementwise expression) folds the same terms
+// again for every output along them: x / sum(x) over f32 [4096, 1000] took
+// 541 us. Here T threads fold each row once, then walk the row's outputs.
+// The fold is bound by HBM; the walk re-reads the row from L2. Same box:
+// 541 -> 11.3 us. From kRowOutputsMinTerms terms on: shorter folds keep one
+// or two threads an output (8192 rows of 10 run in the time of a launch).
+constexpr int64_t kRowOutputsMinTerms = 64;
+
+// The output ranges the reduction does not move with (empty: none).
+std::vector<UOp> row_output_ranges(const KernelInfo& ki) {
+  std::vector<UOp> out;
+  const UOp& R = ki.reduces[0];
+  UOpSet used;
+  for (auto& n : R.toposort())
+    if (n.op() == Op::Range) used.insert(n);
+  int64_t terms = 1;
+  for (size_t i = 1; i < R.srcs().size(); i++) terms *= range_extent(R.src(i));
+  if (terms < kRowOutputsMinTerms) return out;
+  for (size_t i = 0; i < ki.out_ranges.size(); i++)
+    if (!used.count(ki.out_ranges[i]) && ki.out_ext[i] > 1) out.push_back(ki.out_ranges[i]);
+  return out;
+}
+
 // ── RowReduce ───────────────────────────────────────────────────────────────
 RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) {
   const UOp& R = ki.reduces[0];
@@ -1424,13 +1454,18 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   const std::vector<UOp>& ranges = rt.ranges;
   const UOp r_in = ranges.back();
   int64_t L = range_extent(r_in);
-  int T = std::min<int>(256, pow2_floor(std::max<int64_t>(1, L / 16)));
-  int OPW = 256 / T;  // outputs per workgroup
-  int64_t NOUT = total_outputs(ki);
+  // Outputs that share a reduction: NOUT groups (rows) of B.
+  const std::vector<UOp> shared = row_output_ranges(ki);
+  int64_t NOUT = total_outputs(ki), B = 1;
+  for (size_t i = 0; i < ki.out_ranges.size(); i++)
+    if (std::find(shared.begin(), shared.end(), ki.out_ranges[i]) != shared.end()) B *= ki.out_ext[i];
+  NOUT /= B;
+  int T = std::min<int>(256, pow2_floor(std::max<int64_t>(1, shared.empty() ? L / 16 : std::max(L, B) / 8)));
+  int OPW = 256 / T;  // outputs (or rows of them) per workgroup
   // Vector width along r_in: all lane-dependent loads unit-stride and aligned.
   const int V = L % 4 == 0 && row_loads_vec4(rt.value, r_in) ? 4 : 1;
   RowSplit sp;
-  if (L > 0 && row_split(ki, rt, rt.terms / L * ((L + T * V - 1) / (T * V)), &sp)) return render_row_reduce_split(ki, sp, name);
+  if (L > 0 && shared.empty() && row_split(ki, rt, rt.terms / L * ((L + T * V - 1) / (T * V)), &sp)) return render_row_reduce_split(ki, sp, name);
   Emitter em;
   em.set_nontemporal_loads(true);
   em.set_streaming_ranges(ki.out_ranges);
@@ -1445,7 +1480,7 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
     const UOp& ix = ld.src(0).src(1);
     if (!em.depends_on(ix, r_in.get())) continue;
     for (auto& o : ki.out_ranges)
-      if (!em.depends_on(ix, o.get())) shared_rows = true;
+      if (shared.empty() && !em.depends_on(ix, o.get())) shared_rows = true;
   }
   if (shared_rows && grid % 8 == 0) {
     // Workgroups are dispatched round-robin over the 8 XCDs: give each XCD a
@@ -1459,8 +1494,7 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   em.line("const long oid = bid * " + std::to_string(OPW) + " + tid / " + std::to_string(T) + ";");
   em.line("const bool active = oid < " + std::to_string(NOUT) + "L;");
   em.line("const long ocl = active ? oid : 0;");
-  decode_outputs(em, ki, "ocl", UOp());
-  std::string result;
+  decode_outputs(em, ki, "ocl", shared);
   em.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
     FG_CHECK(RR == R, "row reduce renders exactly one reduction");
     std::string acc = "racc";
@@ -1531,9 +1565,49 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
     em.remember_here(RR, lane, acc);
     return acc;
   };
-  std::string v = em.val(ki.value, 0);
-  (void)result;
-  em.line("if (active && rlane == 0) " + pname(ki.out_param) + "[" + em.idx(ki.out_index, 0) + "] = " + v + ";");
+  const std::string out = pname(ki.out_param);
+  if (shared.empty()) {
+    std::string v = em.val(ki.value, 0);
+    em.line("if (active && rlane == 0) " + out + "[" + em.idx(ki.out_index, 0) + "] = " + v + ";");
+  } else {
+    em.val(R, 0);  // folded here, once per row
+    const UOp fast = pick_fast_output(ki);
+    const bool walk_fast = std::find(shared.begin(), shared.end(), fast) != shared.end();
+    const Affine ao = affine_of(ki.out_index);
+    const DType odt = ki.out_param.dtype();
+    int64_t fext = 1;
+    for (size_t i = 0; i < ki.out_ranges.size(); i++)
+      if (ki.out_ranges[i] == fast) fext = ki.out_ext[i];
+    int VB = walk_fast && fext % 4 == 0 ? 4 : 1;
+    bool vstore = VB == 4 && ao.ok && ao.coef(fast) == 1 && ao.c0 % 4 == 0 &&
+                  (odt.kind == DTypeKind::F32 || odt.kind == DTypeKind::I32);
+    for (auto& t : ao.terms)
+      if (t.first != fast && t.second % 4 != 0) vstore = false;
+    em.open_scope("if (active) for (int b = rlane; b < " + std::to_string(B / VB) + "; b += " + std::to_string(T) + ") {", "}");
+    // The fast range innermost, the others in output order.
+    std::string rest = "b";
+    auto take = [&](const UOp& r, int64_t e, int V) {
+      const std::string n = "idx" + std::to_string(r.arg().a);
+      em.line("const int " + n + " = " + rest + " % " + std::to_string(e / V) + (V > 1 ? " * " + std::to_string(V) : "") + ";");
+      rest = "(" + rest + " / " + std::to_string(e / V) + ")";
+      em.define_range(r, n);
+    };
+    if (walk_fast) take(fast, fext, VB);
+    for (size_t i = ki.out_ranges.size(); i-- > 0;)
+      if (ki.out_ranges[i] != fast && std::find(shared.begin(), shared.end(), ki.out_ranges[i]) != shared.end())
+        take(ki.out_ranges[i], ki.out_ext[i], 1);
+    if (VB == 4) em.set_lane_range(fast, 4);
+    std::vector<std::string> vals;
+    for (int u = 0; u < VB; u++) vals.push_back(em.val(ki.value, u));
+    if (vstore) {
+      const std::string vt = odt.kind == DTypeKind::F32 ? "fg_f4" : "fg_i4";
+      em.line("*(" + vt + "*)(" + out + "+" + em.idx(ki.out_index, 0) + ") = " + vt + "{" + vals[0] + ", " + vals[1] + ", " +
+              vals[2] + ", " + vals[3] + "};");
+    } else {
+      for (int u = 0; u < VB; u++) em.line(out + "[" + em.idx(ki.out_index, u) + "] = " + vals[u] + ";");
+    }
+    em.close_scope();
+  }
   RenderedKernel rk;
   rk.name = name;
   rk.kind = kernel_class_name(KernelClass::RowReduce);
