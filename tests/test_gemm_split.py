@@ -1,0 +1,67 @@
+"""The tiled GEMM's bfloat16 split on HIP: operands of any f32 magnitude,
+infinities, NaN, sums past the split's scaled range, and accuracy against the
+rounding of f32 sums, in every orientation of a Linear's products."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gemm_tiles import products
+
+# (B, in, out): ragged rows and columns; k a multiple of 16, of 4 and of neither.
+SHAPES = [(520, 608, 300), (600, 620, 301), (515, 601, 333)]
+
+
+def data(shape, seed):
+    B, fi, fo = shape
+    r = np.random.default_rng(seed)
+    return (r.standard_normal((B, fi)).astype(np.float32), r.standard_normal((fo, fi)).astype(np.float32),
+            r.standard_normal((B, fo)).astype(np.float32))
+
+
+def run(fg, dev, x, w, g):
+    p = products(fg, dev, x, w, g)
+    fg.Tensor.realize_many(list(p.values()))
+    with np.errstate(all="ignore"):
+        x, w, g = (a.astype(np.float64) for a in (x, w, g))
+        ax, aw, ag = np.abs(x), np.abs(w), np.abs(g)
+        want = {"fwd": (x @ w.T, ax @ aw.T), "dx": (g @ w, ag @ aw), "dw": (g.T @ x, ag.T @ ax)}
+    return {k: (t.numpy().astype(np.float64).reshape(want[k][0].shape), *want[k]) for k, t in p.items()}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_split_is_as_accurate_as_f32_sums(fg, hip, shape):
+    for name, (got, want, _) in run(fg, hip, *data(shape, 1)).items():
+        # 620 terms summed one by one in f32 measure about 4.4e-7 here.
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 5e-7, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_operands_of_any_magnitude(fg, hip, shape):
+    x, w, g = data(shape, 2)
+    scale = np.float32(2.0) ** np.arange(-140, -140 + 4 * 64, 4, dtype=np.float32)  # subnormal to 2^112
+    x = (x * scale[np.arange(len(x)) % 64, None]).astype(np.float32)
+    w = (w * np.float32(2.0 ** 3)).astype(np.float32)
+    g = (g * np.float32(2.0 ** -120)).astype(np.float32)
+    for name, (got, want, terms) in run(fg, hip, x, w, g).items():
+        # Each term's products are exact to about 2^-22 and below 2^-149 not at all.
+        bound = 1e-5 * terms + 1024 * 2.0 ** -149
+        assert np.all(np.abs(got - want) <= bound), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_infinities_nan_and_overflow(fg, hip, shape):
+    x, w, g = data(shape, 3)
+    x[5, 7], x[9, 3], x[11, 2] = np.inf, np.nan, -np.inf
+    w[2, 2], w[40, 40] = np.inf, 3.4e38
+    x[300:303] *= np.float32(1e33)  # finite sums of 1e34 and more
+    g[4, 4], g[6, 100] = np.inf, 3.4e38
+    for name, (got, want, terms) in run(fg, hip, x, w, g).items():
+        assert np.array_equal(np.isnan(got), np.isnan(want)), name
+        over = ~np.isnan(want) & (np.abs(want) > 3.3e38)
+        assert np.array_equal(got[over & np.isinf(want)], want[over & np.isinf(want)]), name
+        fine = ~np.isnan(want) & ~over & (terms < 3.3e38)
+        assert np.all(np.abs(got[fine] - want[fine]) <= 1e-5 * terms[fine]), name
