@@ -3160,6 +3160,15 @@ RenderedKernel render_block(const KernelInfo& ki, KernelClass base, const std::s
 // on separate multiplies and adds as on their loads.
 constexpr int64_t kNarrow = 16;
 
+// The rows layout gives a thread four k, so it needs K of about 1024 to occupy
+// its 256 threads. Shorter products run as the one-pass small GEMM (16x16 MFMA
+// tiles), N = 10, event time: K 64, 10,000 rows 13.8 -> 4.1 us, 50,000 rows
+// 61.8 -> 4.6; K 128, 10,000 rows 14.0 -> 4.1; K 256, 20,000 rows 26.5 -> 5.6;
+// K 512, 10,000 rows 15.0 against 6.5, 1000 rows 4.1 either way; K 1024, 4000
+// rows 7.6 against 5.2, 256 rows 4.1 against 4.5; K 2048, 256 rows 4.1 against
+// 7.5.
+constexpr int64_t kNarrowRowsMinK = 512;
+
 struct NarrowPlan {
   bool rows = false;       // the rows layout (else cols)
   UOp rw, rn;              // wide and narrow output ranges
@@ -3720,7 +3729,10 @@ RenderedKernel render_hip(const UOp& kernel, const std::string& name, int force_
       NarrowPlan np;
       FG_CHECK(match_gemm(ki, &g) && narrow_plan(g, &np), "kernel does not match the narrow GEMM pattern");
       if (!np.rows) rk = render_narrow_cols(ki, g, np, sym);
-      else if (narrow_rows_cached_fits(np)) rk = render_narrow_rows_cached(ki, g, np, sym);
+      else if (np.K < kNarrowRowsMinK && gpu_passes().mfma) {
+        rk = render_small_gemm(ki, g, sym);
+        rk.kind = kernel_class_name(k);
+      } else if (narrow_rows_cached_fits(np)) rk = render_narrow_rows_cached(ki, g, np, sym);
       else rk = render_narrow_rows(ki, g, np, sym);
       break;
     }
