@@ -570,6 +570,16 @@ int fg_debug_plan(fg_tensor** roots, int n, int fuse, int render, char* buf, siz
         os << (i ? ", " : "") << "{\"first\": " << firsts[i] << ", \"name\": \"" << pk.name
            << "\", \"grid\": " << pk.grid[0] << ", \"source\": \"" << json_escape(pk.source) << "\"}";
       }
+      // Runs of row kernels that a replayed sequence would launch as one (in
+      // plan order, outside the batches).
+      os << "], \"row_batches\": [";
+      auto rruns = fg::row_batch_runs(all, binfo, in_batch);
+      for (size_t i = 0; i < rruns.size(); i++) {
+        const auto [f, c] = rruns[i];
+        const fg::RenderedKernel bk = fg::render_row_batch({all.begin() + static_cast<long>(f), all.begin() + static_cast<long>(f + c)});
+        os << (i ? ", " : "") << "{\"first\": " << f << ", \"count\": " << c << ", \"name\": \"" << bk.name
+           << "\", \"grid\": " << bk.grid[0] << ", \"source\": \"" << json_escape(bk.source) << "\"}";
+      }
       // Batches that a replayed sequence would run beside an adjacent
       // independent small GEMM or pair (in plan order), and that launch.
       os << "], \"hbatches\": [";

@@ -954,6 +954,59 @@ std::vector<UOp> loads_in(const UOp& v) {
   return out;
 }
 
+std::string block_params(const KernelInfo& ki, std::vector<std::string>* types, std::vector<std::string>* names);
+
+// ── Row kernels ─────────────────────────────────────────────────────────────
+// A kernel whose outermost output range selects a row of its output (row r at
+// elements [r*c, (r+1)*c), c the output's row stride) and of what it reads can
+// run a few rows per workgroup, next to other such kernels in one launch
+// (render_row_batch). kRowBatchMinRows rows at least: fewer leave CUs idle.
+constexpr int64_t kRowBatchMinRows = 512;
+
+// The elements between the rows that index `a` walks with range r: 0 when it
+// does not depend on r, -1 when its other terms can leave the row.
+int64_t row_stride_of(const Affine& a, const UOp& r) {
+  if (!a.ok) return -1;
+  const int64_t c = a.coef(r);
+  int64_t span = a.c0;
+  if (a.c0 < 0 || c < 0) return -1;
+  for (auto& t : a.terms) {
+    if (t.first == r || t.second == 0) continue;
+    if (t.first.op() != Op::Range || t.second < 0) return -1;
+    span += t.second * (range_extent(t.first) - 1);
+  }
+  return c == 0 ? 0 : span < c ? c : -1;
+}
+
+// Fills rk's row fields for the body `code` (of threadIdx.x, row0 and nrows),
+// which computes `rows` rows over ki's outermost range.
+void set_row_body(const KernelInfo& ki, const std::string& name, const std::string& code, int64_t work, RenderedKernel* rk) {
+  std::vector<std::string> names;
+  const std::string params = block_params(ki, &rk->row_types, &names);
+  rk->row_fn = name + "_row";
+  rk->row_src = "__device__ __forceinline__ void " + rk->row_fn + "(" + params + ", int row0, int nrows) {\n" + code + "}\n";
+  rk->rows = ki.out_ext[0];
+  rk->row_work = work;
+  const UOp& r = ki.out_ranges[0];
+  for (auto& [slot, p] : ki.params) {
+    int64_t stride = 0;
+    auto use = [&](const UOp& index) {
+      const int64_t s = row_stride_of(affine_of(index), r);
+      stride = stride == 0 ? s : s == 0 || s == stride ? stride : -1;
+    };
+    if (p == ki.out_param) use(ki.out_index);
+    for (auto& ld : loads_in(ki.value))
+      if (ld.src(0).src(0) == p) use(ld.src(0).src(1));
+    rk->row_stride.push_back(stride);
+  }
+}
+
+// Whether the kernel's outermost output range selects whole rows of its output.
+bool row_kernel(const KernelInfo& ki) {
+  return !ki.out_ranges.empty() && ki.out_ext[0] >= kRowBatchMinRows &&
+         row_stride_of(affine_of(ki.out_index), ki.out_ranges[0]) == total_outputs(ki) / ki.out_ext[0];
+}
+
 // ── Elementwise over a transposed operand ───────────────────────────────────
 // A load whose unit stride lies along another output range than the stores'
 // (a permuted copy, an operand read through a transpose) costs the plain
@@ -1164,6 +1217,37 @@ RenderedKernel render_elementwise(const KernelInfo& ki, const std::string& name)
   rk.source = std::string(kPrelude) + signature(ki, name, kEwThreads) + " {\n" + em.code() + "}\n";
   rk.block[0] = kEwThreads;
   rk.grid[0] = static_cast<unsigned>((threads + kEwThreads - 1) / kEwThreads);
+  if (row_kernel(ki)) {
+    // The same values, a row's outputs (the fast range in vectors) walked by
+    // the workgroup's threads.
+    const int64_t per_row = T / ki.out_ext[0];
+    const int VR = fast != ki.out_ranges[0] ? V : 1;
+    Emitter er;
+    er.open_scope("for (int e = threadIdx.x; e < nrows * " + std::to_string(per_row / VR) + "; e += 256) {", "}");
+    er.line("int rest = e % " + std::to_string(per_row / VR) + ";");
+    er.line("const int idx" + std::to_string(ki.out_ranges[0].arg().a) + " = row0 + e / " + std::to_string(per_row / VR) + ";");
+    er.define_range(ki.out_ranges[0], "idx" + std::to_string(ki.out_ranges[0].arg().a));
+    auto take = [&](const UOp& r, int64_t ext, int v) {
+      const std::string n = "idx" + std::to_string(r.arg().a), es = std::to_string(ext / v);
+      er.line("const int " + n + " = rest % " + es + (v > 1 ? " * " + std::to_string(v) : "") + "; rest /= " + es + ";");
+      er.define_range(r, n);
+    };
+    if (fast != ki.out_ranges[0]) take(fast, fext, VR);
+    for (size_t i = ki.out_ranges.size(); i-- > 1;)
+      if (ki.out_ranges[i] != fast) take(ki.out_ranges[i], ki.out_ext[i], 1);
+    if (VR == 4) er.set_lane_range(fast, 4);
+    std::vector<std::string> rv;
+    for (int u = 0; u < VR; u++) rv.push_back(er.val(ki.value, u));
+    if (vstore && VR == 4) {
+      const char* vt = ki.out_param.dtype().kind == DTypeKind::F32 ? "fg_f4" : "fg_i4";
+      er.line(std::string("*(") + vt + "*)(" + out + "+" + er.idx(ki.out_index, 0) + ") = " + vt + "{" + rv[0] + ", " +
+              rv[1] + ", " + rv[2] + ", " + rv[3] + "};");
+    } else {
+      for (int u = 0; u < VR; u++) er.line(out + "[" + er.idx(ki.out_index, u) + "] = " + rv[u] + ";");
+    }
+    er.close_scope();
+    set_row_body(ki, name, er.code(), per_row, &rk);
+  }
   return rk;
 }
 
@@ -1466,10 +1550,14 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   const int V = L % 4 == 0 && row_loads_vec4(rt.value, r_in) ? 4 : 1;
   RowSplit sp;
   if (L > 0 && shared.empty() && row_split(ki, rt, rt.terms / L * ((L + T * V - 1) / (T * V)), &sp)) return render_row_reduce_split(ki, sp, name);
-  Emitter em;
-  em.set_nontemporal_loads(true);
-  em.set_streaming_ranges(ki.out_ranges);
   const int64_t grid = (NOUT + OPW - 1) / OPW;
+  // The kernel, or with `rows` the body that computes rows [row0, row0 + nrows)
+  // (one group of outputs each) on one workgroup.
+  auto emit = [&](Emitter& em, bool rows) {
+  if (!rows) {
+    em.set_nontemporal_loads(true);
+    em.set_streaming_ranges(ki.out_ranges);
+  }
   em.line("const int tid = threadIdx.x;");
   em.line("const int rlane = tid % " + std::to_string(T) + ";");
   // Whether some streamed operand (one that varies along the reduce axis) is
@@ -1482,7 +1570,11 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
     for (auto& o : ki.out_ranges)
       if (shared.empty() && !em.depends_on(ix, o.get())) shared_rows = true;
   }
-  if (shared_rows && grid % 8 == 0) {
+  if (rows) {
+    em.open_scope("for (int rp = 0; rp < nrows; rp += " + std::to_string(OPW) + ") {", "}");
+    em.line("const bool active = rp + tid / " + std::to_string(T) + " < nrows;");
+    em.line("const long ocl = row0 + (active ? rp + tid / " + std::to_string(T) + " : 0);");
+  } else if (shared_rows && grid % 8 == 0) {
     // Workgroups are dispatched round-robin over the 8 XCDs: give each XCD a
     // contiguous run of outputs, so the outputs that share an input row read
     // it through one L2. (Outputs that each stream their own rows keep the
@@ -1491,9 +1583,11 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   } else {
     em.line("const long bid = blockIdx.x;");
   }
-  em.line("const long oid = bid * " + std::to_string(OPW) + " + tid / " + std::to_string(T) + ";");
-  em.line("const bool active = oid < " + std::to_string(NOUT) + "L;");
-  em.line("const long ocl = active ? oid : 0;");
+  if (!rows) {
+    em.line("const long oid = bid * " + std::to_string(OPW) + " + tid / " + std::to_string(T) + ";");
+    em.line("const bool active = oid < " + std::to_string(NOUT) + "L;");
+    em.line("const long ocl = active ? oid : 0;");
+  }
   decode_outputs(em, ki, "ocl", shared);
   em.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
     FG_CHECK(RR == R, "row reduce renders exactly one reduction");
@@ -1556,12 +1650,14 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
     if (T > 64) {
       int nw = T / 64;
       em.line(std::string("__shared__ ") + ctype(dt) + " fg_part[4];");
+      if (rows) em.line("__syncthreads();");  // the pass before has read it
       em.line("if ((tid & 63) == 0) fg_part[tid >> 6] = " + acc + ";");
       em.line("__syncthreads();");
       em.line("{ const int g0 = (tid >> 6) & ~" + std::to_string(nw - 1) + "; " + acc + " = fg_part[g0];");
       for (int w = 1; w < nw; w++) em.line("  " + acc + " = " + combine(rop, acc, "fg_part[g0+" + std::to_string(w) + "]") + ";");
       em.line("}");
     }
+    if (rows) em.pin_here(RR);
     em.remember_here(RR, lane, acc);
     return acc;
   };
@@ -1608,12 +1704,21 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
     }
     em.close_scope();
   }
+  if (rows) em.close_scope();
+  };
+  Emitter em;
+  emit(em, false);
   RenderedKernel rk;
   rk.name = name;
   rk.kind = kernel_class_name(KernelClass::RowReduce);
   rk.source = std::string(kPrelude) + signature(ki, name, 256) + " {\n" + em.code() + "}\n";
   rk.block[0] = 256;
-  rk.grid[0] = static_cast<unsigned>((NOUT + OPW - 1) / OPW);
+  rk.grid[0] = static_cast<unsigned>(grid);
+  if (row_kernel(ki) && NOUT == ki.out_ext[0]) {
+    Emitter er;
+    emit(er, true);
+    set_row_body(ki, name, er.code(), std::max(rt.terms, B), &rk);
+  }
   return rk;
 }
 
@@ -3760,13 +3865,25 @@ RenderedKernel render_hip(const UOp& kernel, const std::string& name, int force_
 RenderedKernel render_hip_stable(const UOp& kernel) {
   static const std::string kPlaceholder = "FGKERNELNAME";
   RenderedKernel rk = render_hip(kernel, kPlaceholder);
-  uint64_t h = 1469598103934665603ULL;
-  for (unsigned char c : rk.source) {
-    h ^= c;
-    h *= 1099511628211ULL;
-  }
+  auto hash_of = [](const std::string& text) {
+    uint64_t h = 1469598103934665603ULL;
+    for (unsigned char c : text) {
+      h ^= c;
+      h *= 1099511628211ULL;
+    }
+    return static_cast<unsigned long long>(h & 0xffffffffffffULL);
+  };
   char hex[32];
-  std::snprintf(hex, sizeof(hex), "k%012llx", static_cast<unsigned long long>(h & 0xffffffffffffULL));
+  std::snprintf(hex, sizeof(hex), "k%012llx", hash_of(rk.source));
+  if (!rk.row_fn.empty()) {
+    // Kernels of one source can differ in their rows (the outermost range):
+    // the body over rows has its own hash in its name.
+    char own[32];
+    std::snprintf(own, sizeof(own), "%012llx", hash_of(rk.row_src));
+    const std::string fn = rk.row_fn;
+    rk.row_fn += own;
+    rk.row_src.replace(rk.row_src.find(fn + "("), fn.size(), rk.row_fn);
+  }
   auto replace_all = [&](std::string& s) {
     for (size_t p = s.find(kPlaceholder); p != std::string::npos; p = s.find(kPlaceholder, p))
       s.replace(p, kPlaceholder.size(), hex);
@@ -3777,6 +3894,8 @@ RenderedKernel render_hip_stable(const UOp& kernel) {
   replace_all(rk.stage_src);
   replace_all(rk.hbody_fn);
   replace_all(rk.hbody_src);
+  replace_all(rk.row_fn);
+  replace_all(rk.row_src);
   for (auto& l : rk.launches) replace_all(l.func);
   return rk;
 }
@@ -3855,6 +3974,87 @@ RenderedKernel render_block_batch(const std::vector<const RenderedKernel*>& stag
   rk.kind = "block_batch";
   rk.block[0] = kBlockThreads;
   return rk;
+}
+
+RenderedKernel render_row_batch(const std::vector<const RenderedKernel*>& stages) {
+  FG_CHECK(stages.size() >= 2, "a row batch runs at least two kernels");
+  static const std::string kPlaceholder = "FGROWBATCHNAME";
+  const int64_t rows = stages[0]->rows;
+  int64_t work = 1;
+  for (auto* st : stages) {
+    FG_CHECK(!st->row_fn.empty() && st->rows == rows, "kernel " + st->name + " has no body over these rows");
+    work = std::max(work, st->row_work);
+  }
+  // Rows per workgroup: about 4096 elements of the longest row, four
+  // workgroups per CU where there are rows enough.
+  int64_t per = 1;
+  while (per < 64 && 2 * per * work <= 4096 && rows / (2 * per) >= 1024) per *= 2;
+  std::ostringstream src, params, body;
+  src << kPrelude;
+  std::map<std::string, const RenderedKernel*> defined;
+  size_t n = 0;
+  for (size_t i = 0; i < stages.size(); i++) {
+    const RenderedKernel& st = *stages[i];
+    auto [it, fresh] = defined.emplace(st.row_fn, &st);
+    if (fresh) src << st.row_src;
+    else FG_CHECK(it->second->row_src == st.row_src, "render_row_batch: two different bodies named " + st.row_fn);
+    body << (i ? "  __syncthreads();\n  " : "  ") << st.row_fn << "(";
+    for (auto& t : st.row_types) {
+      params << (n ? ", " : "") << t << " a" << n;
+      body << "a" << n++ << ", ";
+    }
+    body << "row0, nrows);\n";
+  }
+  src << "extern \"C\" __global__ void __launch_bounds__(256) " << kPlaceholder << "(" << params.str() << ") {\n"
+      << "  const int row0 = (int)blockIdx.x * " << per << ";\n"
+      << "  const int nrows = " << rows << " - row0 < " << per << " ? " << rows << " - row0 : " << per << ";\n"
+      << body.str() << "}\n";
+  RenderedKernel rk;
+  rk.source = src.str();
+  name_by_hash(rk, kPlaceholder, "rows");
+  rk.kind = "row_batch";
+  rk.block[0] = 256;
+  rk.grid[0] = static_cast<unsigned>((rows + per - 1) / per);
+  return rk;
+}
+
+std::vector<std::pair<size_t, size_t>> row_batch_runs(const std::vector<const RenderedKernel*>& kernels,
+                                                      const std::vector<std::vector<BatchArg>>& args,
+                                                      const std::vector<bool>& excluded) {
+  auto fits = [&](size_t i) {
+    const RenderedKernel& k = *kernels[i];
+    return !excluded[i] && !k.row_fn.empty() && k.launches.empty() && k.scratch_bytes == 0 &&
+           k.row_types.size() == args[i].size() && k.params.size() == args[i].size();
+  };
+  // Whether kernels i and j access what either writes in the same rows only.
+  auto by_row = [&](size_t i, size_t j) {
+    for (size_t a = 0; a < args[i].size(); a++)
+      for (size_t b = 0; b < args[j].size(); b++) {
+        if (!args[i][a].id || args[i][a].id != args[j][b].id) continue;
+        const bool written = kernels[i]->params[a].first == kernels[i]->out_slot || kernels[j]->params[b].first == kernels[j]->out_slot;
+        if (written && (kernels[i]->row_stride[a] <= 0 || kernels[i]->row_stride[a] != kernels[j]->row_stride[b])) return false;
+      }
+    return true;
+  };
+  std::vector<std::pair<size_t, size_t>> runs;
+  for (size_t i = 0; i < kernels.size();) {
+    size_t n = 0, total = 0;
+    if (fits(i)) {
+      n = 1;
+      total = args[i].size();
+      while (i + n < kernels.size() && n < kMaxBatchStages && fits(i + n) && kernels[i + n]->rows == kernels[i]->rows &&
+             total + args[i + n].size() <= FG_MAX_LAUNCH_ARGS) {
+        bool ok = true;
+        for (size_t k = i; k < i + n && ok; k++) ok = by_row(k, i + n);
+        if (!ok) break;
+        total += args[i + n].size();
+        n++;
+      }
+    }
+    if (n >= 2) runs.emplace_back(i, n);
+    i += std::max<size_t>(n, 1);
+  }
+  return runs;
 }
 
 RenderedKernel render_hbatch(const std::vector<const RenderedKernel*>& hb,

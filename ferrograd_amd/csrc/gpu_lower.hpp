@@ -179,6 +179,20 @@ std::vector<HBatchRun> hbatch_runs(const std::vector<const RenderedKernel*>& ker
 std::vector<size_t> pair_runs(const std::vector<const RenderedKernel*>& kernels,
                               const std::vector<std::vector<BatchArg>>& args, const std::vector<bool>& excluded);
 
+// One launch that runs row kernels (RenderedKernel::row_fn, all of the same
+// row count) one after another on a few rows per workgroup, a workgroup
+// barrier between them: each computes exactly what its own kernel computes,
+// and what one leaves for the next stays in the caches of its CU and XCD. The
+// launch takes every kernel's arguments, concatenated.
+RenderedKernel render_row_batch(const std::vector<const RenderedKernel*>& stages);
+// The runs of two or more consecutive row kernels that can share such a
+// launch, as (first, count) pairs: same row count, none marked in `excluded`,
+// at most kMaxBatchStages kernels and FG_MAX_LAUNCH_ARGS arguments, and every
+// buffer one of them writes accessed by the others only in the same rows.
+std::vector<std::pair<size_t, size_t>> row_batch_runs(const std::vector<const RenderedKernel*>& kernels,
+                                                      const std::vector<std::vector<BatchArg>>& args,
+                                                      const std::vector<bool>& excluded);
+
 // The runs of consecutive block kernels a sequence launches as batches, as
 // (first, count) pairs: every run of two or more, split after kMaxBatchStages
 // kernels and before the kernel that would take the run's arguments past

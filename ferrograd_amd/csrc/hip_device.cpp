@@ -292,6 +292,9 @@ class HipDevice : public Device {
       // program, count) and the batch program of each.
       std::vector<std::pair<size_t, size_t>> groups;
       std::vector<std::shared_ptr<Program>> batches;
+      // Runs of consecutive row kernels that launch as one row batch, likewise.
+      std::vector<std::pair<size_t, size_t>> row_groups;
+      std::vector<std::shared_ptr<Program>> row_batches;
       // Pairs of adjacent independent kernels launched together
       // (render_hfused): the first program of each pair, and its launch.
       std::vector<size_t> pair_first;
@@ -330,6 +333,7 @@ class HipDevice : public Device {
         ordered_args.push_back(args[k]);
       }
       group_blocks(ordered, ordered_args, r->groups, r->batches);
+      group_rows(ordered, ordered_args, r->groups, r->row_groups, r->row_batches);
       if (pairs_on()) pair_kernels(ordered, ordered_args, r->groups, r->pair_first, r->pairs);
       if (hbatch_on()) hbatch_kernels(ordered, ordered_args, r->groups, r->pair_first, r->hbatches);
     }
@@ -411,7 +415,7 @@ class HipDevice : public Device {
       nargs.push_back(static_cast<int>(a.size()));
       all.insert(all.end(), a.begin(), a.end());
     };
-    size_t next_group = 0, next_pair = 0, next_hbatch = 0;
+    size_t next_group = 0, next_rows = 0, next_pair = 0, next_hbatch = 0;
     auto append = [&](std::vector<fg_arg>& a, size_t j) {
       std::vector<fg_arg> aj = marshal(static_cast<HipProgram&>(*prog_at(j)), args_at(j));
       a.insert(a.end(), aj.begin(), aj.end());
@@ -454,6 +458,16 @@ class HipDevice : public Device {
         auto& bp = static_cast<HipProgram&>(*r->batches[next_group]);
         add(bp.prog, bp.meta.grid, bp.meta.block, bp.meta.lds_bytes, a);
         next_group++;
+        i += n - 1;
+        continue;
+      }
+      while (next_rows < r->row_groups.size() && r->row_groups[next_rows].first < i) next_rows++;
+      if (next_rows < r->row_groups.size() && r->row_groups[next_rows].first == i) {
+        const size_t n = r->row_groups[next_rows].second;
+        std::vector<fg_arg> a;
+        for (size_t j = i; j < i + n; j++) append(a, j);
+        auto& bp = static_cast<HipProgram&>(*r->row_batches[next_rows]);
+        add(bp.prog, bp.meta.grid, bp.meta.block, bp.meta.lds_bytes, a);
         i += n - 1;
         continue;
       }
@@ -713,6 +727,33 @@ class HipDevice : public Device {
       const BatchForwarding fwd = forwarding_of(progs, args, first, n);
       batches.push_back(compile(render_block_batch(stages, false, forwarding_on() ? &fwd : nullptr), total));
       groups.emplace_back(first, n);
+    }
+  }
+
+  // Runs of two or more consecutive row kernels outside the batches
+  // (row_batch_runs), each compiled into one launch (render_row_batch).
+  void group_rows(const std::vector<Program*>& progs, std::vector<std::vector<KernelArg>>& args,
+                  const std::vector<std::pair<size_t, size_t>>& groups,
+                  std::vector<std::pair<size_t, size_t>>& row_groups, std::vector<std::shared_ptr<Program>>& row_batches) {
+    std::vector<const RenderedKernel*> metas;
+    std::vector<std::vector<BatchArg>> info;
+    std::vector<bool> excluded(progs.size(), false);
+    for (auto [f, c] : groups)
+      for (size_t j = f; j < f + c; j++) excluded[j] = true;
+    for (size_t i = 0; i < progs.size(); i++) {
+      metas.push_back(&progs[i]->meta);
+      info.emplace_back();
+      for (auto& a : args[i])
+        info.back().push_back(a.kind == KernelArg::Kind::Buffer ? BatchArg{a.buffer.get(), a.buffer->numel}
+                                                                 : BatchArg{});
+    }
+    for (auto [first, n] : row_batch_runs(metas, info, excluded)) {
+      std::vector<const RenderedKernel*> stages(metas.begin() + static_cast<long>(first),
+                                                metas.begin() + static_cast<long>(first + n));
+      size_t total = 0;
+      for (size_t j = first; j < first + n; j++) total += args[j].size();
+      row_batches.push_back(compile(render_row_batch(stages), total));
+      row_groups.emplace_back(first, n);
     }
   }
 
