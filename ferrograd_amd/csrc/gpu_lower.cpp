@@ -20,6 +20,7 @@
 #include "gpu_lower.hpp"
 
 #include "../../include/ferrograd_hip.h"
+#include "schedule.hpp"
 
 #include <algorithm>
 #include <charconv>
@@ -115,6 +116,7 @@ KernelInfo analyze_kernel(const UOp& sink) {
     FG_CHECK(sink.src(i).op() == Op::ParamBuffer || sink.src(i).op() == Op::ParamScalar,
              "kernel must be Sink(one effect, kernel parameters)");
   KernelInfo ki;
+  ki.compared = sink.arg().kind == Arg::Kind::Int && sink.arg().a == kComparedSink;
   UOp n = sink.src(0);
   while (n.op() == Op::End) {
     FG_CHECK(n.srcs().size() == 2, "output loop End must carry exactly one body");
@@ -2016,6 +2018,7 @@ std::vector<KmChunk> km_chunks(int T) {
 
 constexpr int64_t kComputeUnits = 256;  // MI355X
 constexpr int kGemmStageK = 16;         // k of one LDS stage of the tiled GEMM, one MFMA deep
+constexpr int kGemmFoldTiles = 5;       // 32x32 tiles of a wave up to which every 2nd stage is folded apart, else every 4th
 constexpr int64_t kLdsPerCu = 163840;   // gfx950 LDS bytes per CU
 constexpr int64_t kMinSplitK = 64;      // shortest K range a split workgroup runs
 
@@ -2042,11 +2045,6 @@ int64_t gemm_tile_residency(const GemmTile& t) {
 //   1024: 369 us as stream-K with eight 32x160 waves (395 with four 64x160),
 //   389 as 256x256 with 4 splits, 368 as 128x256 with 4.
 // - 1000x1001, K 1000: 64x64 28 us, 128x128 with 4 splits 29, 256x256 with 4 46.
-// - A side of at most 32 (N = 10 classes): one operand is streamed once, so the
-//   kernel is HBM-bound: splits up to about two workgroups per CU.
-// - K of at most 32: the kernel is one pass over its output and epilogue
-//   operands. Small tiles put many workgroups' loads and stores in flight
-//   (8192x4096 with K 10, C5's dH2 with the relu mask: 56.8 us with 32x64 tiles).
 // FG_GEMM_TILE="BM,BN,BK,WGM,WGN,S[,NBUF]" fixes the tile, split count (0:
 // stream-K over the chip's CUs) and LDS stage count (2 or 3) of every
 // GEMM in the process: a tuning override for measuring alternatives to the
@@ -2096,6 +2094,10 @@ bool gemm_tile_override(GemmTile* t) {
   return true;
 }
 
+// Products bound by HBM rather than by the matrix cores: the f32 tiles serve
+// them as well (8192x4096 with K 10: 54.8 us, 56.8 on the split ones).
+bool gemm_hbm_bound(int64_t M, int64_t N, int64_t K) { return M <= 32 || N <= 32 || K <= 32; }
+
 GemmTile choose_gemm_tile(int64_t M, int64_t N, int64_t K) {
   auto tiles = [&](const GemmTile& t) { return ((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN); };
   const int64_t smax = std::max<int64_t>(1, K / kMinSplitK);
@@ -2126,21 +2128,6 @@ GemmTile choose_gemm_tile(int64_t M, int64_t N, int64_t K) {
              "FG_GEMM_TILE: stream-K needs at least one k-tile per workgroup");
     return as_stream_k(forced);
   }
-  if (M <= 32 || N <= 32) {
-    GemmTile t;
-    auto side = [](int64_t ext, int* b, int* w) {
-      if (ext <= 32) { *b = 32; *w = 1; }
-      else if (ext >= 256) { *b = 256; *w = 4; }
-      else if (ext >= 128) { *b = 128; *w = 4; }
-      else { *b = 64; *w = 2; }
-    };
-    side(M, &t.BM, &t.WGM);
-    side(N, &t.BN, &t.WGN);
-    t.BK = 16;
-    const int64_t nt = tiles(t);
-    return with_splits(t, std::max<int64_t>(1, std::min(smax, (2 * kComputeUnits + nt - 1) / nt)));
-  }
-  if (K <= 32) return with_splits(GemmTile{32, 64, K <= 16 ? 16 : 32, 1, 2}, 1);
   // Estimated time of each tile and split: rounds of resident workgroups, each
   // an overhead (first loads, epilogue) and its 16-k stages at the time a stage
   // takes with that many workgroups on a CU (one column per workgroup); plus
@@ -2207,6 +2194,146 @@ GemmTile choose_gemm_tile(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+// ── The f32 MFMA tiles (render_gemm_f32) ──
+// Workgroups of a tile one CU holds at once: bounded by the LDS of the two
+// double-buffered operand stages (rows padded by 4 floats) and by the
+// accumulators (16 VGPRs per 32x32 tile, about 128 more for staging and
+// addresses, 512 per SIMD lane).
+int64_t gemm_tile_residency_f32(const GemmTile& t) {
+  const int64_t lds = t.nbuf * 4 * static_cast<int64_t>(t.BM + t.BN + 8) * (t.BK + 4);
+  const int64_t waves_per_simd = std::max<int64_t>(1, 512 / (16 * t.tm() * t.tn() + 128));
+  const int64_t by_waves = std::max<int64_t>(1, waves_per_simd * 4 / (t.WGM * t.WGN));
+  return std::max<int64_t>(1, std::min(kLdsPerCu / lds, by_waves));
+}
+
+// Tile and K splits. Measured on MI355X (fp32, same box and run for each
+// comparison):
+// - MFMA-bound shapes: 256x256 with four 128x128 waves and BK 32 ran 4096^3 at
+//   134.8-137.6 TFLOP/s (hipBLASLt 138.9-142.8), 256x128 and 128x256 at 129,
+//   128x128 at 127. The shape, k-tile and split count are chosen by estimated time:
+//   rounds of resident workgroups times the MFMA time of one tile's K range
+//   (padding included, at each shape's measured efficiency), plus the traffic
+//   of split-K partials; or, for stream-K, each workgroup's share of the
+//   k-tiles plus one more epilogue. For dW1 of the C5 MLP (4096x784, K 8192)
+//   that picks 256x160 tiles as stream-K (410 + 13 us in the train step), over
+//   256x160 with 3 splits on 240 CUs (430 + 10 us) and 256x256 with 4 splits
+//   (484 + 14 us).
+// - A side of at most 32 (N = 10 classes): one operand is streamed once, so the
+//   kernel is HBM-bound. BK 16 (less LDS, more resident workgroups) and splits
+//   up to about two workgroups per CU: the 8192x10 (K 4096) forward took 59 us
+//   with BK 32 and 8 splits, 45 with BK 16 and 16 splits.
+// - K of at most 32: the kernel is one pass over its output and epilogue
+//   operands. Small tiles put many workgroups' loads and stores in flight:
+//   8192x4096 with K 10 (C5's dH2, relu mask) took 91 us with 256x256 tiles, 54
+//   with 128x128, 50 with 64x64; in a later same-box run 53.5 with 64x64 (four
+//   waves), 51.5 with 32x64 (two), 52-53 with 128x64, 58 with 64x128 and 32x32,
+//   65 with 64x32.
+GemmTile choose_gemm_tile_f32(int64_t M, int64_t N, int64_t K) {
+  auto tiles = [&](const GemmTile& t) { return ((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN); };
+  const int64_t smax = std::max<int64_t>(1, K / kMinSplitK);
+  auto with_splits = [&](GemmTile t, int64_t S) {
+    t.KC = ((K + S - 1) / S + t.BK - 1) / t.BK * t.BK;
+    t.S = (K + t.KC - 1) / t.KC;
+    return t;
+  };
+  // Stream-K on every resident workgroup slot of the chip.
+  auto as_stream_k = [&](GemmTile t) {
+    const int64_t kt = (K + t.BK - 1) / t.BK;
+    t.stream_k = true;
+    t.G = kComputeUnits * gemm_tile_residency_f32(t);
+    t.S = stream_k_segments(tiles(t), kt, t.G);
+    t.KC = t.BK;
+    return t;
+  };
+  // Worth it when every workgroup runs at least 4 k-tiles and the shares do
+  // not fall on whole tiles anyway.
+  auto stream_k_fits = [&](const GemmTile& t) {
+    const int64_t kt = (K + t.BK - 1) / t.BK, G = kComputeUnits * gemm_tile_residency_f32(t), iters = tiles(t) * kt;
+    return iters >= 4 * G && !(iters % G == 0 && (iters / G) % kt == 0);
+  };
+  GemmTile forced;
+  if (gemm_tile_override(&forced)) {
+    if (forced.S != 0) return with_splits(forced, forced.S);
+    FG_CHECK(tiles(forced) * ((K + forced.BK - 1) / forced.BK) >= kComputeUnits * gemm_tile_residency_f32(forced),
+             "FG_GEMM_TILE: stream-K needs at least one k-tile per workgroup");
+    return as_stream_k(forced);
+  }
+  if (M <= 32 || N <= 32) {
+    GemmTile t;
+    auto side = [](int64_t ext, int* b, int* w) {
+      if (ext <= 32) { *b = 32; *w = 1; }
+      else if (ext >= 256) { *b = 256; *w = 4; }
+      else if (ext >= 128) { *b = 128; *w = 4; }
+      else { *b = 64; *w = 2; }
+    };
+    side(M, &t.BM, &t.WGM);
+    side(N, &t.BN, &t.WGN);
+    t.BK = 16;
+    const int64_t nt = tiles(t);
+    return with_splits(t, std::max<int64_t>(1, std::min(smax, (2 * kComputeUnits + nt - 1) / nt)));
+  }
+  if (K <= 32) return with_splits(GemmTile{32, 64, K <= 16 ? 16 : 32, 1, 2}, 1);
+  constexpr double kCuFlops = 157.3e12 / kComputeUnits;  // fp32 MFMA peak per CU
+  constexpr double kHbmBytes = 5.0e12;                   // sustained HBM rate for split partials
+  struct Cand {
+    GemmTile t;
+    double eff;  // measured throughput relative to 256x256
+  };
+  // Each shape with BK 32 and BK 16. BK 16 pads a K that is not a multiple of
+  // 32 less: the 8192x4096 forward with K 784 (49 k-tiles of 16) took 399 us
+  // against 424 us with BK 32; for K 4096 BK 32 was about 2% faster.
+  // 256x160 (four waves of 64x160 stacked along M, five 32-wide MFMA columns
+  // each) pads a 784-wide side to 800 columns instead of 1024. C5's dW1
+  // (4096x784, K 8192), timed alone: 472 us with 3 splits (240 workgroups)
+  // against 526 us as 256x256 with 4; with BK 16 (two or three stages) 548 us.
+  const Cand cands[] = {{{256, 256, 32, 2, 2}, 1.0},   {{256, 256, 16, 2, 2}, 0.99}, {{256, 128, 32, 2, 2}, 0.9},
+                        {{256, 128, 16, 2, 2}, 0.89},  {{128, 256, 32, 2, 2}, 0.9},  {{128, 256, 16, 2, 2}, 0.89},
+                        {{128, 128, 32, 2, 2}, 0.92},  {{128, 128, 16, 2, 2}, 0.91}, {{64, 64, 32, 2, 2}, 0.6},
+                        {{256, 160, 32, 4, 1}, 0.97},  {{256, 160, 16, 4, 1}, 0.84}, {{160, 256, 32, 1, 4}, 0.97},
+                        {{160, 256, 16, 1, 4}, 0.84}};
+  GemmTile best = with_splits(GemmTile{64, 64, 32, 2, 2}, 1);
+  double best_s = 1e30;
+  for (const Cand& c : cands) {
+    if (M < c.t.BM / 2 || N < c.t.BN / 2) continue;  // mostly padding
+    const int64_t nt = tiles(c.t), res = gemm_tile_residency_f32(c.t);
+    for (int64_t s = 1; s <= smax; s++) {
+      const GemmTile t = with_splits(c.t, s);
+      if (t.S != s) continue;
+      const int64_t rounds = (nt * t.S + kComputeUnits * res - 1) / (kComputeUnits * res);
+      const double mfma = static_cast<double>(rounds * res) * 2.0 * t.BM * t.BN * t.KC / (kCuFlops * c.eff);
+      const double partials = t.S > 1 ? static_cast<double>(t.S + 1) * M * N * 4.0 / kHbmBytes : 0.0;
+      if (mfma + partials < best_s * 0.999) {
+        best_s = mfma + partials;
+        best = t;
+      }
+    }
+    if (stream_k_fits(c.t)) {
+      // Each workgroup's share of the k-tiles, plus one more epilogue when it
+      // crosses into a second tile, plus the segments' partials.
+      const GemmTile t = as_stream_k(c.t);
+      const int64_t kt = (K + t.BK - 1) / t.BK, share = (nt * kt + t.G - 1) / t.G;
+      const double mfma = static_cast<double>(share + 1) * res * 2.0 * t.BM * t.BN * t.BK / (kCuFlops * c.eff);
+      const double partials = static_cast<double>(t.S + 1) * M * N * 4.0 / kHbmBytes;
+      if (mfma + partials < best_s * 0.98) {
+        best_s = mfma + partials;
+        best = t;
+      }
+    }
+  }
+  // A 16-wide k-tile runs with three LDS stages where they fit without costing
+  // a resident workgroup: its k-tiles are half as long, so the read of the next
+  // stage's first fragments after each barrier weighed twice as much. Measured
+  // on the 8192x4096 forward with K 784: 455-462 us against 463-464 us with two
+  // stages; 4096^3 with BK 16: 1054 against 1071 us (BK 32, two stages: 1034).
+  if (best.BK == 16) {
+    GemmTile t3 = best;
+    t3.nbuf = 3;
+    const int64_t lds3 = 3 * 4 * static_cast<int64_t>(t3.BM + t3.BN + 8) * (t3.BK + 4);
+    if (lds3 <= kLdsPerCu && gemm_tile_residency_f32(t3) == gemm_tile_residency_f32(best)) best = t3;
+  }
+  return best;
+}
+
 constexpr int64_t kSmallGemmMaxWork = int64_t(1) << 26;  // M*N*K
 constexpr int kSmallGemmMaxGroups = 4;                   // 16-k groups per wave
 
@@ -2262,7 +2389,7 @@ bool match_gemm(const KernelInfo& ki, GemmMatch* g) {
   if (g->M <= 32 || g->N <= 32) {
     // A narrow product pays for a 32-wide MFMA tile only when the grid fills
     // the chip; otherwise the row and column reductions serve it better.
-    GemmTile t = choose_gemm_tile(g->M, g->N, g->K);
+    GemmTile t = choose_gemm_tile_f32(g->M, g->N, g->K);
     if (((g->M + t.BM - 1) / t.BM) * ((g->N + t.BN - 1) / t.BN) * t.S < 128) return false;
   }
   return true;
@@ -2392,6 +2519,111 @@ RenderedKernel render_small_gemm(const KernelInfo& ki, const GemmMatch& g, const
   return rk;
 }
 
+// Helpers of the generated f32 GEMM: vector types for 1/2/4 operands per LDS read
+// and the instruction interleave of one k-tile (sched_group_barrier masks:
+// 0x008 MFMA, 0x020 VMEM read, 0x100 DS read, 0x200 DS write). Group g's MFMAs
+// are paired one to one with the global loads of the next stage (group 0), the
+// LDS reads of group g+1, and the LDS writes of the next stage (last group), so
+// those instructions issue while the MFMA pipe is busy.
+const char* kGemmF32Prelude = R"(typedef float fg_f2 __attribute__((ext_vector_type(2)));
+template <int V> struct fg_vt;
+template <> struct fg_vt<1> { typedef float t; };
+template <> struct fg_vt<2> { typedef fg_f2 t; };
+template <> struct fg_vt<4> { typedef fg_f4 t; };
+template <int mask, int n>
+__device__ __forceinline__ void fg_sched_pairs() {
+  if constexpr (n > 0) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(mask, 1, 0);
+    fg_sched_pairs<mask, n - 1>();
+  }
+}
+template <int G, int g, int NV, int ND, int NW, int MF>
+__device__ __forceinline__ void fg_sched_k_tile() {
+  constexpr int nv = g == 0 ? NV : 0, nd = g + 1 < G ? ND : 0, nw = g == G - 1 ? NW : 0;
+  constexpr int rest = MF - nv - nd - nw;
+  fg_sched_pairs<0x020, nv>();
+  fg_sched_pairs<0x100, nd>();
+  fg_sched_pairs<0x200, nw>();
+  if constexpr (rest > 0) __builtin_amdgcn_sched_group_barrier(0x008, rest, 0);
+  if constexpr (g + 1 < G) fg_sched_k_tile<G, g + 1, NV, ND, NW, MF>();
+}
+)";
+
+// The k loop with three LDS operand stages instead of two: the stage after
+// next is written while a stage is computed, so the next stage was complete
+// at the previous barrier and its first fragments are read during the last
+// group's MFMAs, before the barrier, instead of after it. One barrier per
+// k-tile still orders every write after the reads of the stage it replaces
+// (read during the k-tile before the last barrier) and before its own reads
+// (after the next barrier). Needs an even number of 8-k groups per k-tile, so
+// the fragment registers of the next k-tile's first group are free.
+std::string gemm_three_stages(std::string src) {
+  auto swap_once = [&](const std::string& from, const std::string& to) {
+    const size_t p = src.find(from);
+    FG_CHECK(p != std::string::npos && src.find(from, p + 1) == std::string::npos,
+             "three-stage GEMM: generated text not found once");
+    src.replace(p, from.size(), to);
+  };
+  swap_once("  // Operand stages, double-buffered, rows padded by 4 floats;",
+            "  // Operand stages, three of them, rows padded by 4 floats;");
+  swap_once("constexpr int SA = 2 * SA_R * SA_C, SB = 2 * SB_R * SB_C,",
+            "constexpr int SA = 3 * SA_R * SA_C, SB = 3 * SB_R * SB_C,");
+  swap_once("__device__ __forceinline__ void fg_sched_k_tile() {\n"
+            "  constexpr int nv = g == 0 ? NV : 0, nd = g + 1 < G ? ND : 0, nw = g == G - 1 ? NW : 0;",
+            "__device__ __forceinline__ void fg_sched_k_tile() {\n"
+            "  constexpr int nv = g == 0 ? NV : 0, nd = ND, nw = g == G - 1 ? NW : 0;");
+  swap_once(R"(  load_a(kbeg); load_b(kbeg);
+  store_a(0, kbeg); store_b(0, kbeg);
+  __syncthreads();
+  frag(0, 0, fa[0], fb[0]);
+  for (int kt = 0; kt < KT; kt++) {
+    const int cur = kt & 1;
+    // The last k-tile reloads itself, so the body is the same every time.
+    const int knext = kbeg + (kt + 1 < KT ? kt + 1 : kt) * BK;
+    load_a(knext); load_b(knext);
+    #pragma unroll
+    for (int g = 0; g < BK / 8; g++) {
+      if (g + 1 < BK / 8) frag(cur, g + 1, fa[(g + 1) & 1], fb[(g + 1) & 1]);
+)",
+            R"(  static_assert((BK / 8) % 2 == 0, "three stages need an even number of 8-k groups");
+  load_a(kbeg); load_b(kbeg);
+  store_a(0, kbeg); store_b(0, kbeg);
+  {
+    const int k1 = kbeg + (1 < KT ? 1 : 0) * BK;
+    load_a(k1); load_b(k1);
+    store_a(1, k1); store_b(1, k1);
+  }
+  __syncthreads();
+  frag(0, 0, fa[0], fb[0]);
+  int cur = 0;
+  for (int kt = 0; kt < KT; kt++) {
+    const int nxt = cur == 2 ? 0 : cur + 1, nn = nxt == 2 ? 0 : nxt + 1;
+    // The last k-tiles reload the last one, so the body is the same every time.
+    const int knext = kbeg + (kt + 2 < KT ? kt + 2 : KT - 1) * BK;
+    load_a(knext); load_b(knext);
+    #pragma unroll
+    for (int g = 0; g < BK / 8; g++) {
+      if (g + 1 < BK / 8) frag(cur, g + 1, fa[(g + 1) & 1], fb[(g + 1) & 1]);
+      else frag(nxt, 0, fa[0], fb[0]);
+)");
+  swap_once(R"(      if (g == BK / 8 - 1) { store_a(cur ^ 1, knext); store_b(cur ^ 1, knext); }
+    }
+    fg_sched_k_tile<BK / 8, 0, NV_, ND_, NW_, 4 * TM * TN>();
+    __syncthreads();
+    frag(cur ^ 1, 0, fa[0], fb[0]);
+  }
+)",
+            R"(      if (g == BK / 8 - 1) { store_a(nn, knext); store_b(nn, knext); }
+    }
+    fg_sched_k_tile<BK / 8, 0, NV_, ND_, NW_, 4 * TM * TN>();
+    __syncthreads();
+    cur = nxt;
+  }
+)");
+  return src;
+}
+
 // Helpers of the generated GEMM: the split of f32 values into three bfloat16
 // parts (see render_gemm) and the MFMA over them.
 const char* kGemmPrelude = R"(typedef float fg_f2 __attribute__((ext_vector_type(2)));
@@ -2496,6 +2728,533 @@ int64_t stream_k_tile_period(int64_t ntiles, int64_t kt, int64_t G) {
   return 0;
 }
 
+// ── Tiled GEMM on the f32 MFMA ──────────────────────────────────────────────
+// For two kinds of products; the others run on the split tiles below.
+// - Products a comparison of the same schedule reads (KernelInfo::compared, a
+//   layer's output under relu in a train step). Two correct f32 orders put a
+//   value within rounding of zero on either side, and the mask then takes or
+//   drops whole terms of the gradient: after a second step of the
+//   784-4096-4096-10 MLP the logits of this order and of the split one were
+//   up to 4.5e-6 apart (one of 20 seeds), with these products left to this
+//   order 2e-7. They cost C5's step 1.1 ms (5,534 us against 4,426).
+// - Products bound by HBM (gemm_hbm_bound).
+RenderedKernel render_gemm_f32(const KernelInfo& ki, const GemmMatch& g, const std::string& name) {
+  const int64_t M = g.M, N = g.N, K = g.K;
+  const GemmTile tile = choose_gemm_tile_f32(M, N, K);
+  const int BM = tile.BM, BN = tile.BN, BK = tile.BK, WGM = tile.WGM, WGN = tile.WGN, NT = tile.nt();
+  const int TM = tile.tm(), TN = tile.tn();
+  const int64_t S = tile.S, KC = tile.KC, NP = (N + 3) / 4 * 4;
+  const int64_t ntiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  FG_CHECK(BM % (32 * WGM) == 0 && BN % (32 * WGN) == 0 && BK % 8 == 0, "gemm tile shape does not fit the wave grid");
+  FG_CHECK(TM >= 1 && TM <= 5 && TN >= 1 && TN <= 5, "gemm wave tile must be 32 to 160 wide");
+  FG_CHECK(tile.nbuf == 2 || (tile.nbuf == 3 && (BK / 8) % 2 == 0), "three GEMM stages need an even number of 8-k groups");
+  const bool split = S > 1 || tile.stream_k;  // partials in scratch, summed by _fin
+  const int64_t KTT = (K + BK - 1) / BK;       // k-tiles per tile
+  const int64_t sk_D = tile.stream_k ? stream_k_tile_period(ntiles, KTT, tile.G) : 0;
+  const std::string scratch_param = split ? ", float* __restrict__ fg_scratch" : "";
+  const int waves_per_eu = static_cast<int>(std::max<int64_t>(1, gemm_tile_residency_f32(tile) * NT / 256));
+  auto sig = [&](const std::string& fn, int block, bool main) {
+    std::string s = signature(ki, fn, block);
+    s = s.substr(0, s.size() - 1) + scratch_param + ")";
+    if (main) {
+      const std::string lb = "__launch_bounds__(" + std::to_string(block) + ") ";
+      s.replace(s.find(lb), lb.size(),
+                lb + "__attribute__((amdgpu_waves_per_eu(" + std::to_string(waves_per_eu) + "))) ");
+    }
+    return s;
+  };
+  const std::string main_name = split ? name + "_part" : name;
+
+  // How each operand reaches LDS. Mode 0: 4 consecutive k per thread (unit
+  // stride along k: 16-byte loads), staged [row][k]. Mode 1: 4 consecutive rows
+  // per thread (unit stride along m/n), staged [k][row] with the rows of tile i
+  // interleaved (tile i row r is wave row T*r+i), so one LDS read gives a lane
+  // its operand for all T tiles. Mode 2: one element per load, staged along
+  // whichever index moves faster in memory.
+  struct Stage {
+    int md = 2;
+    bool km = false;
+    int groups = 0, per = 0, V = 1;
+    bool k_fast = true;
+    std::vector<UOp> lds;
+  };
+  auto plan = [&](const GemmOperand& op, int BX, int64_t ext) {
+    Stage st;
+    const int64_t so = op.lead.coef(op.rout), sk = op.lead.coef(g.rk);
+    if (sk == 1 && K % 4 == 0) st.md = 0;
+    else if (so == 1 && ext % 4 == 0) st.md = 1;
+    st.k_fast = std::llabs(sk) <= std::llabs(so);
+    st.km = st.md == 1 || (st.md == 2 && !st.k_fast);
+    st.V = st.md == 2 ? 1 : 4;
+    st.groups = st.md == 2 ? BX * BK : BX * BK / 4;
+    st.per = (st.groups + NT - 1) / NT;
+    st.lds = loads_in(op.expr);
+    return st;
+  };
+  const Stage sa = plan(g.a, BM, M), sb = plan(g.b, BN, N);
+  const int NV = sa.per * static_cast<int>(sa.lds.size()) + sb.per * static_cast<int>(sb.lds.size());
+  const int ND = (sa.km ? 4 * static_cast<int>(km_chunks(TM).size()) : TM) +
+                 (sb.km ? 4 * static_cast<int>(km_chunks(TN).size()) : TN);
+  const int NW = sa.per + sb.per;
+
+  std::ostringstream s;
+  s << kPrelude << kGemmF32Prelude;
+  s << "#define M_ " << M << "\n#define N_ " << N << "\n#define K_ " << K << "\n#define NP_ " << NP << "\n";
+  s << "#define S_ " << S << "\n#define KC_ " << KC << "\n#define NTILES_ " << ntiles << "\n";
+  s << "#define BM " << BM << "\n#define BN " << BN << "\n#define BK " << BK << "\n";
+  s << "#define NT " << NT << "\n#define WGN " << WGN << "\n#define TM " << TM << "\n#define TN " << TN << "\n";
+  s << "#define A_KM " << (sa.km ? 1 : 0) << "\n#define B_KM " << (sb.km ? 1 : 0) << "\n";
+  s << "#define NV_ " << NV << "\n#define ND_ " << ND << "\n#define NW_ " << NW << "\n";
+  if (tile.stream_k) {
+    s << "#define G_ " << tile.G << "\n#define KTT_ " << KTT << "\n#define ITERS_ " << ntiles * KTT << "L\n";
+    if (sk_D > 0) s << "#define SK_D_ " << sk_D << "\n";
+    s << "// Stream-K: the workgroup that runs (tile, k-tile) iteration x.\n"
+         "__device__ __forceinline__ int fg_sk_owner(long x) { return (int)(((x + 1) * G_ - 1) / ITERS_); }\n";
+  }
+  s << sig(main_name, NT, true) << " {\n";
+  s << R"(  // Operand stages, double-buffered, rows padded by 4 floats; then per-wave
+  // 32 x WN staging tiles for the epilogue.
+  constexpr int WM = BM / (NT / 64 / WGN), WN = BN / WGN;
+  // A [row][k] stage of 16-wide k-tiles is unpadded, its 16-byte chunks
+  // XOR-swizzled by row: chunk c of row r sits at c ^ ((r >> 2) & 3). The 16
+  // lanes a fragment read serves at once (16 rows, one chunk, over 64 banks)
+  // and the 8 lanes of a stage write (two rows, over 32) then fall on distinct
+  // banks: PMC SQ_LDS_BANK_CONFLICT 0 for C5's K = 784 forward, against
+  // 6.5e6 cycles per dispatch with rows padded to 20 floats (which put two
+  // rows' writes on the same banks) and with c ^ ((r >> 1) & 3) (which put
+  // rows r and r + 8 of a read on the same banks).
+#define FG_SWZ(r, c) (BK == 16 ? ((c) ^ ((((r) >> 2) & 3) << 2)) : (c))
+#if A_KM
+  constexpr int SA_R = BK, SA_C = BM + 4;
+#else
+  constexpr int SA_R = BM, SA_C = BK == 16 ? BK : BK + 4;
+#endif
+#if B_KM
+  constexpr int SB_R = BK, SB_C = BN + 4;
+#else
+  constexpr int SB_R = BN, SB_C = BK == 16 ? BK : BK + 4;
+#endif
+  constexpr int SA = 2 * SA_R * SA_C, SB = 2 * SB_R * SB_C, EPS = WN + 4, SE = (NT / 64) * 32 * EPS;
+  __shared__ __attribute__((aligned(16))) float smem[(SA + SB) > SE ? (SA + SB) : SE];
+  float (*As)[SA_R][SA_C] = reinterpret_cast<float (*)[SA_R][SA_C]>(smem);
+  float (*Bs)[SB_R][SB_C] = reinterpret_cast<float (*)[SB_R][SB_C]>(smem + SA);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, r32 = lane & 31;
+  const int nbm = (M_ + BM - 1) / BM, nbn = (N_ + BN - 1) / BN;
+  int bid = blockIdx.x;
+  // Blocks are dispatched round-robin over the 8 XCDs; give each XCD a
+  // contiguous run of (split, tile) pairs so neighbouring tiles of one K
+  // range share its L2.
+  if ((NTILES_ * S_) % 8 == 0) bid = (bid % 8) * (NTILES_ * S_ / 8) + bid / 8;
+#if S_ > 1
+  const int ks = bid / NTILES_;
+  bid = bid % NTILES_;
+  const int kbeg = ks * KC_, kend = (kbeg + KC_ < K_) ? kbeg + KC_ : K_;
+#else
+  constexpr int kbeg = 0, kend = K_;
+#endif
+  const int GM = 8;
+  const int group = bid / (GM * nbn), first_m = group * GM;
+  const int gsz = (nbm - first_m) < GM ? (nbm - first_m) : GM;
+  const int tm = first_m + (bid % (GM * nbn)) % gsz, tn = (bid % (GM * nbn)) / gsz;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
+  floatx16 acc[TM][TN];
+  #pragma unroll
+  for (int i = 0; i < TM; i++)
+    #pragma unroll
+    for (int j = 0; j < TN; j++)
+      #pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+)";
+  // Global -> register loaders. load_X issues the operand's raw loads; store_X
+  // evaluates the operand expression (relu recompute, masks) on them when it
+  // writes the next stage to LDS, late in the k-tile, so the loads stay in
+  // flight under the MFMAs. Out-of-range elements load from a clamped, valid
+  // address and are replaced by 0 with a select: the k-tile body has no
+  // branches, so its instructions can be interleaved as one region.
+  std::set<std::string> rsrc_declared;
+  auto loader = [&](const char* X, const GemmOperand& op, const Stage& st, int BX, int64_t ext, const char* dim) {
+    const int V = st.V, per = st.per;
+    const bool guard = st.groups % NT != 0;
+    // Bounds checks only where a tile can overhang: rows when the extent is not
+    // a multiple of the tile, k when K is not a multiple of BK (the K splits
+    // are multiples of BK). Statically in-range loads keep their plain
+    // addresses, which saves registers in the large tiles.
+    const bool row_check = ext % BX != 0, k_check = K % BK != 0;
+    // Raw buffer loads where every load of the operand allows them: a 32-bit
+    // byte offset per lane that is the same in every k-tile, and the k-tile's
+    // start in the scalar offset, so the k loop computes no addresses and
+    // holds one register per load instead of a 64-bit address. Each load must
+    // read a 4-byte element of a buffer under 2 GiB at an affine index whose
+    // terms are all ranges or constants with non-negative coefficients (the
+    // per-lane part is then a valid offset on its own; a kernel scalar, such
+    // as a narrow() start, could be negative for all the renderer knows), and
+    // k must need no bounds check (the k-tile's start is not clamped). Measured on C5's kernels alone (same box, same bits): the
+    // 8192x4096, K 4096 products 1.4-2.0% faster (forward with the relu of its
+    // input, dH with the relu mask, dW with the SGD update), dW1's stream-K
+    // pass 1.7%, the K 784 forward within 0.6%.
+    bool bufl = !k_check;
+    for (auto& ld : st.lds) {
+      const UOp& ix = ld.src(0);
+      const DTypeKind dk = ld.dtype().kind;
+      if (dk != DTypeKind::F32 && dk != DTypeKind::I32) bufl = false;
+      if (ix.src(0).op() != Op::ParamBuffer || ix.src(0).arg().b * 4 >= (int64_t(1) << 31)) bufl = false;
+      Affine a = affine_of(ix.src(1));
+      if (!a.ok || a.c0 < 0) bufl = false;
+      for (auto& t : a.terms)
+        if (t.second < 0 || t.first.op() != Op::Range) bufl = false;
+    }
+    std::map<const UOpInner*, std::string> rsrc;
+    std::ostringstream decl;
+    if (bufl)
+      for (auto& ld : st.lds) {
+        const UOp& pb = ld.src(0).src(0);
+        const std::string nm = "fg_rs_" + pname(pb);
+        rsrc[pb.get()] = nm;
+        if (rsrc_declared.insert(nm).second)
+          decl << "  const __amdgpu_buffer_rsrc_t " << nm << " = __builtin_amdgcn_make_buffer_rsrc((void*)" << pname(pb)
+               << ", (short)0, " << pb.arg().b * 4 << ", 0x00020000);\n";
+      }
+    auto reg = [&](size_t i, const std::string& slot) { return "r" + std::string(X) + std::to_string(i) + "[" + slot + "]"; };
+    auto slot = [&](int u) { return V == 1 ? std::string("j") : "4*j+" + std::to_string(u); };
+    auto coords = [&]() {
+      std::ostringstream c;
+      c << "      const int idx = tid + NT * j;\n";
+      if (st.md == 0) c << "      const int r = idx / (BK / 4), kk = (idx % (BK / 4)) * 4;\n";
+      else if (st.md == 1) c << "      const int kk = idx / (" << BX << " / 4), r = (idx % (" << BX << " / 4)) * 4;\n";
+      else if (st.k_fast) c << "      const int r = idx / BK, kk = idx % BK;\n";
+      else c << "      const int kk = idx / " << BX << ", r = idx % " << BX << ";\n";
+      c << "      const int gr = " << dim << "0 + r, gk = k0 + kk;\n";
+      std::string cond;
+      if (guard) cond += "idx < " + std::to_string(st.groups);
+      if (row_check) cond += (cond.empty() ? "" : " && ") + std::string("gr < ") + std::to_string(ext);
+      if (k_check) cond += (cond.empty() ? "" : " && ") + std::string("gk < kend");
+      if (cond.empty()) {
+        c << "      constexpr bool in = true;\n      const int grc = gr, gkc = gk;\n";
+      } else {
+        c << "      const bool in = " << cond << ";\n";
+        c << "      const int grc = in ? gr : 0, gkc = in ? gk : 0;\n";
+      }
+      return c.str();
+    };
+    auto setup = [&](Emitter& em, bool loads) {
+      // 64-bit index arithmetic: the per-j address offsets are then constants
+      // the compiler folds into the loads, instead of 32-bit sums it must
+      // recompute and sign-extend (which alone cost 80+ spilled VGPRs in the
+      // 256x256 tile).
+      em.define_range(op.rout, "(long)grc");
+      if (loads && bufl) {
+        em.define_range(g.rk, "(long)kk");
+        em.set_buffer_loads(rsrc, g.rk, "k0");
+      } else {
+        em.define_range(g.rk, "(long)gkc");
+      }
+      if (st.md == 0) em.set_lane_range(g.rk, 4);
+      else if (st.md == 1) em.set_lane_range(op.rout, 4);
+    };
+    auto indent = [](const std::string& code, const char* pre) {
+      std::ostringstream o;
+      std::istringstream is(code);
+      std::string ln;
+      while (std::getline(is, ln)) o << pre << ln << "\n";
+      return o.str();
+    };
+    std::ostringstream l;
+    l << decl.str();
+    for (size_t i = 0; i < st.lds.size(); i++)
+      l << "  " << ctype(st.lds[i].dtype()) << " r" << X << i << "[" << per * V << "];\n";
+    l << "  auto load_" << X << " = [&](int k0) {\n";
+    l << "    #pragma unroll\n    for (int j = 0; j < " << per << "; j++) {\n" << coords();
+    {
+      Emitter em;
+      setup(em, true);
+      std::ostringstream body;
+      for (size_t i = 0; i < st.lds.size(); i++)
+        for (int u = 0; u < V; u++) body << reg(i, slot(u)) << " = " << em.val(st.lds[i], u) << ";\n";
+      l << indent(em.code() + body.str(), "      ");
+    }
+    l << "    }\n  };\n";
+    const char* SX = X[0] == 'a' ? "As" : "Bs";
+    l << "  auto store_" << X << " = [&](int buf, int k0) {\n";
+    l << "    #pragma unroll\n    for (int j = 0; j < " << per << "; j++) {\n" << coords();
+    {
+      Emitter em;
+      setup(em, false);
+      em.load_cb_ = [&](const UOp& ld, int u) -> std::string {
+        for (size_t i = 0; i < st.lds.size(); i++)
+          if (st.lds[i] == ld) return reg(i, slot(u));
+        return std::string();
+      };
+      std::vector<std::string> vals;
+      for (int u = 0; u < V; u++) vals.push_back(em.val(op.expr, u));
+      std::ostringstream body;
+      for (int u = 0; u < V; u++) body << "v[" << u << "] = in ? " << vals[u] << " : 0.0f;\n";
+      l << "      float v[" << V << "];\n";
+      if (!(st.lds.size() == 1 && op.expr == st.lds[0])) {
+        // The operand is an expression of its loads (a relu recomputed, a
+        // mask): pass the raw registers through an empty asm here, so the
+        // expression's instructions cannot be scheduled ahead of this point.
+        // Without it the scheduler put some of them right after the k-tile's
+        // first loads, each behind a wait for those loads to arrive: the C5
+        // forward with relu(H) as its operand ran 1990 us against 1830 us for
+        // the plain product of the same shape.
+        std::string regs;
+        for (size_t i = 0; i < st.lds.size(); i++)
+          for (int u = 0; u < V; u++) regs += (regs.empty() ? "" : ", ") + std::string("\"+v\"(") + reg(i, slot(u)) + ")";
+        l << "      asm volatile(\"\" : " << regs << ");\n";
+      }
+      l << indent(em.code() + body.str(), "      ");
+    }
+    const std::string sguard = guard ? "if (idx < " + std::to_string(st.groups) + ") " : "";
+    if (st.md == 0) {
+      l << "      " << sguard << "*(fg_f4*)(&" << SX << "[buf][r][FG_SWZ(r, kk)]) = fg_f4{v[0], v[1], v[2], v[3]};\n";
+    } else if (st.md == 1) {
+      l << "      " << sguard << "*(fg_f4*)(&" << SX << "[buf][kk][r]) = fg_f4{v[0], v[1], v[2], v[3]};\n";
+    } else if (st.km) {
+      l << "      " << sguard << SX << "[buf][kk][r] = v[0];\n";
+    } else {
+      l << "      " << sguard << SX << "[buf][r][FG_SWZ(r, kk)] = v[0];\n";
+    }
+    l << "    }\n  };\n";
+    return l.str();
+  };
+  s << loader("a", g.a, sa, BM, M, "m");
+  s << loader("b", g.b, sb, BN, N, "n");
+  // [k][row] stages: one LDS read of each chunk's interleaved rows per MFMA step.
+  auto km_frag = [&](const char* stage, const char* w, const char* fr, int T) {
+    std::ostringstream f;
+    f << "    #pragma unroll\n    for (int t = 0; t < 4; t++) {\n";
+    for (const KmChunk& c : km_chunks(T)) {
+      f << "      {\n        const typename fg_vt<" << c.size << ">::t v = *(const typename fg_vt<" << c.size
+        << ">::t*)&" << stage << "[buf][8 * g + 4 * h + t][" << w << " + " << 32 * c.first << " + " << c.size
+        << " * r32];\n";
+      f << "        #pragma unroll\n        for (int i = 0; i < " << c.size << "; i++) " << fr << "[" << c.first
+        << " + i][t] = ((const float*)&v)[i];\n      }\n";
+    }
+    f << "    }\n";
+    return f.str();
+  };
+  // Wave-block position of row r of tile i in a [k][row] stage.
+  auto km_pos = [&](int T, const std::string& i, const std::string& r) {
+    std::string e = "0";
+    const auto ch = km_chunks(T);
+    for (size_t c = ch.size(); c-- > 0;) {
+      const std::string here = std::to_string(32 * ch[c].first) + " + " + std::to_string(ch[c].size) + " * " + r +
+                               " + (" + i + " - " + std::to_string(ch[c].first) + ")";
+      e = c + 1 == ch.size() ? here : "(" + i + " < " + std::to_string(ch[c].first + ch[c].size) + " ? " + here + " : " + e + ")";
+    }
+    return e;
+  };
+  // Epilogue staging of a [k][row] B operand's columns: one LDS write per chunk.
+  auto km_stage = [&]() {
+    std::ostringstream f;
+    for (const KmChunk& c : km_chunks(TN)) {
+      f << "      {\n        typename fg_vt<" << c.size << ">::t v;\n";
+      f << "        #pragma unroll\n        for (int j = 0; j < " << c.size << "; j++) ((float*)&v)[j] = acc[i]["
+        << c.first << " + j][e];\n";
+      f << "        *(typename fg_vt<" << c.size << ">::t*)(wst + rr * EPS + " << 32 * c.first << " + " << c.size
+        << " * r32) = v;\n      }\n";
+    }
+    return f.str();
+  };
+  s << R"(  // K schedule: in group g (8 k), MFMA step t, lane half h uses k = 8g + 4h + t.
+  float fa[2][TM][4], fb[2][TN][4];
+  auto frag = [&](int buf, int g, float (&fra)[TM][4], float (&frb)[TN][4]) {
+#if A_KM
+)" << km_frag("As", "wm", "fra", TM) << R"(#else
+    #pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const fg_f4 v = *(const fg_f4*)&As[buf][wm + 32 * i + r32][FG_SWZ(wm + 32 * i + r32, 8 * g + 4 * h)];
+      fra[i][0] = v.x; fra[i][1] = v.y; fra[i][2] = v.z; fra[i][3] = v.w;
+    }
+#endif
+#if B_KM
+)" << km_frag("Bs", "wn", "frb", TN) << R"(#else
+    #pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const fg_f4 v = *(const fg_f4*)&Bs[buf][wn + 32 * j + r32][FG_SWZ(wn + 32 * j + r32, 8 * g + 4 * h)];
+      frb[j][0] = v.x; frb[j][1] = v.y; frb[j][2] = v.z; frb[j][3] = v.w;
+    }
+#endif
+  };
+  const int KT = (kend - kbeg + BK - 1) / BK;
+  load_a(kbeg); load_b(kbeg);
+  store_a(0, kbeg); store_b(0, kbeg);
+  __syncthreads();
+  frag(0, 0, fa[0], fb[0]);
+  for (int kt = 0; kt < KT; kt++) {
+    const int cur = kt & 1;
+    // The last k-tile reloads itself, so the body is the same every time.
+    const int knext = kbeg + (kt + 1 < KT ? kt + 1 : kt) * BK;
+    load_a(knext); load_b(knext);
+    #pragma unroll
+    for (int g = 0; g < BK / 8; g++) {
+      if (g + 1 < BK / 8) frag(cur, g + 1, fa[(g + 1) & 1], fb[(g + 1) & 1]);
+      #pragma unroll
+      for (int t = 0; t < 4; t++)
+        #pragma unroll
+        for (int i = 0; i < TM; i++)
+          #pragma unroll
+          for (int j = 0; j < TN; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[g & 1][i][t], fb[g & 1][j][t], acc[i][j], 0, 0, 0);
+      if (g == BK / 8 - 1) { store_a(cur ^ 1, knext); store_b(cur ^ 1, knext); }
+    }
+    fg_sched_k_tile<BK / 8, 0, NV_, ND_, NW_, 4 * TM * TN>();
+    __syncthreads();
+    frag(cur ^ 1, 0, fa[0], fb[0]);
+  }
+  // Epilogue: each wave stages the 32 x WN accumulators of tile row i in its
+  // own LDS tile (32x32 MFMA layout: element e of lane l is row
+  // 8*(e/4) + 4*(l/32) + e%4, column l%32 of its tile), then reads them back as
+  // rows of float4, so epilogue operands load and outputs store 16 bytes per
+  // lane.
+  __syncthreads();
+  float* wst = smem + wave * (32 * EPS);
+  #pragma unroll
+  for (int i = 0; i < TM; i++) {
+    #pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int rr = 8 * (e >> 2) + 4 * h + (e & 3);
+#if B_KM
+)" << km_stage() << R"(#else
+      #pragma unroll
+      for (int j = 0; j < TN; j++) wst[rr * EPS + 32 * j + r32] = acc[i][j][e];
+#endif
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int q = 0; q < WN / 8; q++) {
+      const int ch = lane + 64 * q, rr = ch / (WN / 4), cc = (ch % (WN / 4)) * 4;
+      const fg_f4 gv = *(const fg_f4*)(wst + rr * EPS + cc);
+#if A_KM
+      const int grow = m0 + wm + )" << km_pos(TM, "i", "rr") << R"(;
+#else
+      const int grow = m0 + wm + 32 * i + rr;
+#endif
+      const int gcol = n0 + wn + cc;
+      if (grow < M_ && gcol < N_) {
+)";
+  // Everything outside the reduction, for the four columns gcol..gcol+3 of
+  // row grow whose sums are in gv.
+  auto epilogue = [&]() {
+    static const char* kComp[4] = {"gv.x", "gv.y", "gv.z", "gv.w"};
+    Emitter em;
+    em.define_range(g.rm, "grow");
+    const std::string out = pname(ki.out_param);
+    if (N % 4 == 0) {
+      // Every column group lies inside the tile: lanes along the columns.
+      em.define_range(g.rn, "gcol");
+      em.set_lane_range(g.rn, 4);
+      em.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
+        FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
+        return kComp[lane];
+      };
+      std::vector<std::string> vals;
+      for (int u = 0; u < 4; u++) vals.push_back(em.val(ki.value, u));
+      Affine ao = affine_of(ki.out_index);
+      bool vstore = ao.ok && ao.coef(g.rn) == 1 && ao.c0 % 4 == 0 &&
+                    ki.out_param.dtype().kind == DTypeKind::F32;
+      for (auto& t : ao.terms)
+        if (t.first != g.rn && t.second % 4 != 0) vstore = false;
+      if (vstore) {
+        em.line("*(float4*)(" + out + "+" + em.idx(ki.out_index, 0) + ") = make_float4(" + vals[0] + ", " + vals[1] +
+                ", " + vals[2] + ", " + vals[3] + ");");
+      } else {
+        for (int u = 0; u < 4; u++) em.line(out + "[" + em.idx(ki.out_index, u) + "] = " + vals[u] + ";");
+      }
+    } else {
+      // Ragged last column group: one guarded column at a time.
+      for (int u = 0; u < 4; u++) {
+        const std::string col = "(gcol+" + std::to_string(u) + ")";
+        em.open_scope("if (" + col + " < N_) {", "}");
+        em.define_range(g.rn, col);
+        em.reduce_cb_ = [&, u](const UOp& RR, int) -> std::string {
+          FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
+          return kComp[u];
+        };
+        std::string v = em.val(ki.value, 0);
+        em.line(out + "[" + em.idx(ki.out_index, 0) + "] = " + v + ";");
+        em.close_scope();
+      }
+    }
+    return em.code();
+  };
+  auto indent = [](const std::string& code, const std::string& pre) {
+    std::ostringstream o;
+    std::istringstream is(code);
+    std::string l;
+    while (std::getline(is, l)) o << pre << l << "\n";
+    return o.str();
+  };
+  if (!split) {
+    s << indent(epilogue(), "        ");
+  } else {
+    // Raw partial sums of this K range; the epilogue runs after they are summed.
+    s << "        *(fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol) = gv;\n";
+  }
+  s << "      }\n    }\n    __syncthreads();\n  }\n";
+  if (tile.stream_k) s << "  }\n";  // the workgroup's next segment
+  s << "}\n";
+  if (split) {
+    // Second pass: one thread per 4 columns of a row sums the partials in
+    // split order (stream-K: the tile's segments, in k order), then runs the
+    // epilogue.
+    s << sig(name + "_fin", 256, false) << " {\n";
+    s << R"(  const long gid = (long)blockIdx.x * 256 + threadIdx.x;
+  if (gid >= (long)M_ * (NP_ / 4)) return;
+  const int grow = (int)(gid / (NP_ / 4)), gcol = (int)(gid % (NP_ / 4)) * 4;
+  fg_f4 gv = *(const fg_f4*)(fg_scratch + (long)grow * NP_ + gcol);
+)";
+    if (tile.stream_k && sk_D > 0) {
+      // The tile's block index (the inverse of the main pass's row-major
+      // slot), then how many workgroups its k-tiles were split over.
+      s << R"(  const int nbn = (N_ + BN - 1) / BN, sq = (grow / BM) * nbn + gcol / BN;
+  const long t0 = (long)((sq % (NTILES_ / SK_D_)) * SK_D_ + sq / (NTILES_ / SK_D_)) * KTT_;
+  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
+  for (int ks = 1; ks < nseg; ks++) {)";
+    } else if (tile.stream_k) {
+      // The tile's block index (the inverse of the main pass's grouped
+      // order), then how many workgroups its k-tiles were split over.
+      s << R"(  const int nbm = (M_ + BM - 1) / BM, nbn = (N_ + BN - 1) / BN, GM = 8;
+  const int tm = grow / BM, tn = gcol / BN, group = tm / GM, first_m = group * GM;
+  const int gsz = (nbm - first_m) < GM ? (nbm - first_m) : GM;
+  const long t0 = (long)(group * GM * nbn + tn * gsz + (tm - first_m)) * KTT_;
+  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
+  for (int ks = 1; ks < nseg; ks++) {)";
+    } else {
+      s << "  for (int ks = 1; ks < S_; ks++) {";
+    }
+    s << R"(
+    const fg_f4 p = *(const fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol);
+    gv.x = gv.x + p.x; gv.y = gv.y + p.y; gv.z = gv.z + p.z; gv.w = gv.w + p.w;
+  }
+  if (gcol < N_) {
+)";
+    s << indent(epilogue(), "    ");
+    s << "  }\n}\n";
+  }
+  RenderedKernel rk;
+  rk.name = name;
+  rk.kind = kernel_class_name(KernelClass::Gemm);
+  rk.source = s.str();
+  if (tile.nbuf == 3) rk.source = gemm_three_stages(rk.source);
+  rk.block[0] = static_cast<unsigned>(NT);
+  rk.grid[0] = static_cast<unsigned>(tile.stream_k ? tile.G : ntiles * S);
+  if (tile.stream_k) rk.source = gemm_stream_k(rk.source, sk_D);
+  if (split) {
+    LaunchSpec a, b;
+    a.func = name + "_part";
+    a.grid[0] = rk.grid[0];
+    a.block[0] = static_cast<unsigned>(NT);
+    b.func = name + "_fin";
+    b.grid[0] = static_cast<unsigned>((M * (NP / 4) + 255) / 256);
+    b.block[0] = 256;
+    rk.launches = {a, b};
+    rk.scratch_bytes = static_cast<size_t>(S * M * NP) * sizeof(float);
+  }
+  return rk;
+}
+
 // ── Tiled GEMM on the bfloat16 matrix cores, at f32 precision ──────────────
 // The f32 MFMA runs at 157 TFLOP/s and bound the large products (91-95% of
 // it); the bfloat16 MFMA runs 16 times as fast. Every f32 value is the exact
@@ -2510,19 +3269,26 @@ int64_t stream_k_tile_period(int64_t ntiles, int64_t kt, int64_t G) {
 // NaN, |sum| of 2^96 and more) is computed again with the f32 MFMA from the
 // operands in memory.
 //
-// Error against 64 bits (2-norm, normal data, one K range): K 784 4.3e-7 (f32
-// MFMA 5.0e-7), K 4096 1.0e-6 (1.14e-6), K 8192 1.4e-6 (1.6e-6); relu(x)-like
-// data, K 4096, 5.3e-7 (8.4e-7). Fewer roundings per sum (six per 16 k against
-// eight) more than pay for the dropped terms.
+// Error against 64 bits (2-norm): the six products are added to the running
+// sums one after another, smallest first, except in every 2nd stage (waves of
+// few tiles) or 4th, whose products are summed apart and added once. The
+// bfloat16 MFMA rounds the aligned sum down, so the operands' odd rows are
+// negated and the results' signs alternate: without that the errors of all
+// sums leaned the same way (mean -2.1e-7 of their spread at K 4096, 1e-10
+// with). 4096^3: 8.8e-7 (f32 MFMA 1.1e-6); 3000x1500x1001 forward, input and
+// weight gradient 2.6e-7, 2.6e-7, 2.7e-7 (3.1e-7, 4.0e-7, 4.4e-7); K 8192
+// 1.4e-6 or less (1.6e-6).
 //
-// 4096^3 (4096 outputs, bias): 948 -> 621 us a call, 221 TFLOP/s; C5's train
-// step 7,052 -> 4,409 us. What bounds it: power and the matrix pipe. The same
-// loop without the split ran at 242 TFLOP/s, without loads, split and LDS
-// writes at 259 (register-only bfloat16 MFMAs on the same data: 267-310).
-// Adding each stage's six products into a zeroed accumulator and that into the
-// sum (error 3.1e-7 at K 4096) cost 9%.
+// 4096^3 with bias: 948 -> 625 us a call, 220 TFLOP/s. What bounds it is power
+// and the matrix pipe (70% busy at 1.88 GHz of 2.4): the same loop without the
+// split ran at 242 TFLOP/s, without loads, split and LDS writes at 259;
+// register-only bfloat16 MFMAs on the same data at 267-310. Loads two stages
+// ahead, wave priorities, 4 waves of 128x128 (196-200) and sched_group_barrier
+// interleaving did not help. Summing every stage's products apart (error
+// 3.1e-7) cost 9-11%, every 4th 0-4%.
 RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::string& name) {
   if (small_gemm_fits(g.M, g.N, g.K)) return render_small_gemm(ki, g, name);
+  if (ki.compared || gemm_hbm_bound(g.M, g.N, g.K)) return render_gemm_f32(ki, g, name);
   const int64_t M = g.M, N = g.N, K = g.K;
   const GemmTile tile = choose_gemm_tile(M, N, K);
   const int BM = tile.BM, BN = tile.BN, BK = tile.BK, WGM = tile.WGM, WGN = tile.WGN, NT = tile.nt();
@@ -2568,9 +3334,8 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     return st;
   };
   const Stage sa = plan(g.a, BM), sb = plan(g.b, BN);
-  const bool k_short = K < kGemmStageK;                    // one stage, its k past K clamped one by one
   const bool k_inner = BK % kGemmStageK != 0;              // a split's k range can end inside a stage
-  const bool k_ragged = !k_short && (K % kGemmStageK != 0 || k_inner);  // the last stage is read from K - 16 on
+  const bool k_ragged = K % kGemmStageK != 0 || k_inner;   // the last stage is read from K - 16 on
 
   std::ostringstream s;
   s << kPrelude << kGemmPrelude;
@@ -2578,7 +3343,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
   s << "#define S_ " << S << "\n#define KC_ " << KC << "\n#define NTILES_ " << ntiles << "\n";
   s << "#define BM " << BM << "\n#define BN " << BN << "\n#define BK " << BK << "\n";
   s << "#define NT " << NT << "\n#define WGN " << WGN << "\n#define TM " << TM << "\n#define TN " << TN << "\n";
-  s << "#define NBUF_ " << tile.nbuf << "\n";
+  s << "#define NBUF_ " << tile.nbuf << "\n#define FOLD_ " << (TM * TN <= kGemmFoldTiles ? 2 : 4) << "\n";
   if (tile.stream_k) {
     s << "#define G_ " << tile.G << "\n#define KTT_ " << KTT << "\n#define ITERS_ " << ntiles * KTT << "L\n";
     if (sk_D > 0) s << "#define SK_D_ " << sk_D << "\n";
@@ -2654,7 +3419,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     // terms are all ranges or constants with non-negative coefficients (the
     // per-lane part is then a valid offset on its own; a kernel scalar, such
     // as a narrow() start, could be negative for all the renderer knows).
-    bool bufl = !k_short;
+    bool bufl = true;
     for (auto& ld : st.lds) {
       const UOp& ix = ld.src(0);
       const DTypeKind dk = ld.dtype().kind;
@@ -2701,17 +3466,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     };
     l << "  auto load_" << X << " = [&](fg_raw& w, int k0) {\n" << k0c;
     l << "    #pragma unroll\n    for (int j = 0; j < " << st.per << "; j++) {\n" << coords;
-    if (k_short) {
-      for (int u = 0; u < V; u++) {
-        Emitter em;
-        const std::string us = std::to_string(u);
-        em.define_range(op.rout, "(long)grc");
-        em.define_range(g.rk, "(long)(kk + " + us + " < K_ ? kk + " + us + " : K_ - 1)");
-        std::ostringstream body;
-        for (size_t i = 0; i < st.lds.size(); i++) body << reg(i, u) << " = " << em.val(st.lds[i], 0) << ";\n";
-        l << "      {\n" << indent(em.code() + body.str(), "        ") << "      }\n";
-      }
-    } else {
+    {
       Emitter em;
       setup(em, true);
       std::ostringstream body;
@@ -2736,12 +3491,11 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       for (int u = 0; u < V; u++) {
         const std::string k = "kk + " + std::to_string(u);
         std::string in;
-        if (k_short) in = k + " < K_";
         if (k_ragged) in = "k0c + " + k + " >= k0";
         if (k_inner) in += (in.empty() ? "" : " && ") + std::string("k0c + ") + k + " < kend";
-        body << "v[" << u << "] = " << vals[u] << " * " << (in.empty() ? "65536.0f" : "(" + in + " ? 65536.0f : 0.0f)") << ";\n";
+        body << "v[" << u << "] = " << vals[u] << " * " << (in.empty() ? "sc" : "(" + in + " ? sc : 0.0f)") << ";\n";
       }
-      l << "      float v[" << V << "];\n";
+      l << "      const float sc = (r & 1) ? -65536.0f : 65536.0f;\n      float v[" << V << "];\n";
       if (!(st.lds.size() == 1 && op.expr == st.lds[0])) {
         // The operand is an expression of its loads (a relu recomputed, a
         // mask): pass the raw registers through an empty asm here, so the
@@ -2784,13 +3538,26 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     #pragma unroll
     for (int q = 0; q < 3; q++) f[q] = *(const fg_i4*)(smem + buf * STG + 6 * PLA + (2 * q + h) * PLB + (wn + 32 * j + r32) * 16);
   };
-  // The six products of a column of tiles, smallest first.
-  auto mac = [&](int j, const fg_i4 (&a)[TM][3], const fg_i4 (&b)[3]) {
+  // The six products of a column of tiles, smallest first. A stage with `fold`
+  // sums them apart: one rounding of the running sums instead of six.
+  auto mac = [&](bool fold, int j, const fg_i4 (&a)[TM][3], const fg_i4 (&b)[3]) {
     constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
-    #pragma unroll
-    for (int t = 0; t < 6; t++)
+    if (fold) {
       #pragma unroll
-      for (int i = 0; i < TM; i++) acc[i][j] = fg_mfma(a[i][pa[t]], b[pb[t]], acc[i][j]);
+      for (int i = 0; i < TM; i++) {
+        floatx16 t;
+        #pragma unroll
+        for (int e = 0; e < 16; e++) t[e] = 0.0f;
+        #pragma unroll
+        for (int q = 0; q < 6; q++) t = fg_mfma(a[i][pa[q]], b[pb[q]], t);
+        acc[i][j] += t;
+      }
+    } else {
+      #pragma unroll
+      for (int q = 0; q < 6; q++)
+        #pragma unroll
+        for (int i = 0; i < TM; i++) acc[i][j] = fg_mfma(a[i][pa[q]], b[pb[q]], acc[i][j]);
+    }
   };
   const int KT = (kend - kbeg + 15) / 16;
   auto kat = [&](int t) { return kbeg + (t < KT ? t : KT - 1) * 16; };  // past the last stage: it again
@@ -2813,7 +3580,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
   frag_a(0, fa);
   frag_b(0, 0, fb[0]);
   int cur = 0;
-  for (int kt = 0; kt < KT; kt++) {
+  auto stage = [&](bool fold, int kt) {
     const int nxt = cur == 2 ? 0 : cur + 1, aft = nxt == 2 ? 0 : nxt + 1;
     fg_i4 fn[TM][3];
     store_a(w, aft, kat(kt + 2)); store_b(w, aft, kat(kt + 2));
@@ -2823,7 +3590,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       if (j + 1 < TN) frag_b(cur, j + 1, fb[(j + 1) & 1]);
       else frag_b(nxt, 0, fb[(j + 1) & 1]);
       if (j == TN - 2 || TN == 1) frag_a(nxt, fn);
-      mac(j, fa, fb[j & 1]);
+      mac(fold, j, fa, fb[j & 1]);
     }
     __syncthreads();
     #pragma unroll
@@ -2835,13 +3602,13 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       for (int q = 0; q < 3; q++) fb[0][q] = fb[1][q];
     }
     cur = nxt;
-  }
+  };
 #else
   load_a(w, kat(0)); load_b(w, kat(0));
   store_a(w, 0, kat(0)); store_b(w, 0, kat(0));
   load_a(w, kat(1)); load_b(w, kat(1));
   __syncthreads();
-  for (int kt = 0; kt < KT; kt++) {
+  auto stage = [&](bool fold, int kt) {
     const int cur = kt & 1;
     fg_i4 fa[TM][3], fb[2][3];
     frag_a(cur, fa);
@@ -2851,11 +3618,22 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     #pragma unroll
     for (int j = 0; j < TN; j++) {
       if (j + 1 < TN) frag_b(cur, j + 1, fb[(j + 1) & 1]);
-      mac(j, fa, fb[j & 1]);
+      mac(fold, j, fa, fb[j & 1]);
     }
     __syncthreads();
+  };
+#endif
+  int kt = 0;
+#if FOLD_ > 1
+  #pragma unroll 1
+  for (; kt + FOLD_ <= KT; kt += FOLD_) {
+    stage(true, kt);
+    #pragma unroll
+    for (int f = 1; f < FOLD_; f++) stage(false, kt + f);
   }
 #endif
+  #pragma unroll 1
+  for (; kt < KT; kt++) stage(FOLD_ == 1, kt);
   // Sums that are not finite (infinite operands, overflow of the scaled sums)
   // are computed again from the f32 operands, one 32x32 tile at a time.
   float chk = 0.0f;
@@ -2868,6 +3646,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
   if (chk != chk) fg_bad = 1;
   __syncthreads();
   const bool again = fg_bad != 0;
+  const float descale = r32 & 1 ? -0x1p-32f : 0x1p-32f;  // row and column signs
   auto f32_tile = [&](int i, int j) {
     const int ra = m0 + wm + 32 * i + r32, rb = n0 + wn + 32 * j + r32;
     const int rac = ra < M_ ? ra : M_ - 1, rbc = rb < N_ ? rb : N_ - 1;
@@ -2893,7 +3672,9 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     const int i = ij / (WN / EW), jj = ij % (WN / EW);
     #pragma unroll
     for (int j = 0; j < EW / 32; j++) {
-      floatx16 t = acc[i][jj * (EW / 32) + j] * 0x1p-32f;
+      floatx16 t = acc[i][jj * (EW / 32) + j];
+      #pragma unroll
+      for (int e = 0; e < 16; e++) t[e] *= e & 1 ? -descale : descale;
       if (again) t = f32_tile(i, jj * (EW / 32) + j);
       #pragma unroll
       for (int e = 0; e < 16; e++) wst[(8 * (e >> 2) + 4 * h + (e & 3)) * EPS + 32 * j + r32] = t[e];

@@ -30,6 +30,7 @@ struct KernelInfo {
   std::vector<int64_t> out_ext;
   std::vector<UOp> reduces;     // Reduce nodes in the stored value
   std::vector<std::pair<int, UOp>> params;  // slot -> ParamBuffer / ParamScalar
+  bool compared = false;  // a comparison of the same schedule reads the output (kComparedSink)
 };
 KernelInfo analyze_kernel(const UOp& sink);
 int64_t range_extent(const UOp& r);

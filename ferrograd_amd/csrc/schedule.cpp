@@ -113,7 +113,7 @@ std::pair<UOp, std::vector<KernelArg>> parameterize_inputs(const UOp& root, size
 }
 
 // schedule.rs:131-151
-ScheduleItem parameterize(const UOp& expr, const ScheduleOptions& opt) {
+ScheduleItem parameterize(const UOp& expr, const ScheduleOptions& opt, bool compared) {
   Device& backend = get_device(expr.device());
   auto [p, inputs] = parameterize_inputs(expr, 1, opt);
   Shape out_shape;
@@ -122,7 +122,7 @@ ScheduleItem parameterize(const UOp& expr, const ScheduleOptions& opt) {
   UOp out_param = UOp::param_buffer(0, expr.dtype(), static_cast<int64_t>(numel(out_shape)), expr.device());
   UOp store = UOp::make_new(Op::Store, DType::Void(), {out_param, p}, Arg::none());
   ScheduleItem item;
-  item.sink = UOp::sink({store});
+  item.sink = compared ? UOp::make_new(Op::Sink, DType::Void(), {store}, Arg::integer(kComparedSink)) : UOp::sink({store});
   item.inputs = std::move(inputs);
   item.output_buffer = out;
   item.out_shape = out_shape;
@@ -388,6 +388,23 @@ UOp identity_copy_source(const UOp& node) {
   return row_major(shape, strides) ? b : UOp();
 }
 
+// Whether a comparison reads `node`, directly or through views.
+bool feeds_comparison(const UOp& node, const UOpMap<std::vector<UOp>>& consumers) {
+  std::vector<UOp> stack{node};
+  UOpSet seen;
+  while (!stack.empty()) {
+    const UOp n = stack.back();
+    stack.pop_back();
+    auto it = consumers.find(n);
+    if (!seen.insert(n).second || it == consumers.end()) continue;
+    for (auto& c : it->second) {
+      if (c.op() == Op::CmpLt) return true;
+      if (is_movement(c.op())) stack.push_back(c);
+    }
+  }
+  return false;
+}
+
 bool is_held(const UOp& node, const ScheduleOptions& opt) {
   return opt.held && opt.held->get(node.get()) != PtrIndexMap::kAbsent;
 }
@@ -534,7 +551,7 @@ SchedulePlan schedule_many(const std::vector<UOp>& exprs, const ScheduleOptions&
   SchedulePlan plan;
   auto materialize = [&](const UOp& node) {
     UOp kexpr = substitute_materialized(node, plan.replacements);
-    ScheduleItem item = parameterize(kexpr, opt);
+    ScheduleItem item = parameterize(kexpr, opt, opt.fuse && feeds_comparison(node, consumers));
     plan.replacements[node] = buffer_replacement(item);
     plan.items.push_back(std::move(item));
   };
@@ -625,7 +642,7 @@ SchedulePlan schedule_many(const std::vector<UOp>& exprs, const ScheduleOptions&
       plan.items.push_back(parameterize_store(store, opt));
       plan.replacements[expr] = value;
     } else {
-      ScheduleItem item = parameterize(fin, opt);
+      ScheduleItem item = parameterize(fin, opt, opt.fuse && feeds_comparison(expr, consumers));
       plan.replacements[expr] = buffer_replacement(item);
       plan.items.push_back(std::move(item));
     }

@@ -29,6 +29,22 @@ def run(fg, dev, x, w, g):
     return {k: (t.numpy().astype(np.float64).reshape(want[k][0].shape), *want[k]) for k, t in p.items()}
 
 
+def test_products_a_comparison_reads_keep_the_f32_mfma(fg, cpu):
+    """A train step's hidden layers feed relu masks; their input and weight
+    gradients, and a product nothing compares, are split."""
+    t = lambda *s: fg.Tensor.new(np.ones(s, np.float32), list(s), cpu)  # noqa: E731
+    w1, w2 = t(700, 600).with_requires_grad(True), t(650, 700).with_requires_grad(True)
+    x = t(640, 600)
+    z1 = x.matmul(w1.permute([1, 0]))
+    z2 = z1.relu().matmul(w2.permute([1, 0]))
+    grads = z2.mul(t(640, 650)).sum([0, 1]).gradient([w1, w2])
+    items = fg.debug_plan([z2, *grads], fuse=True, render_hip=True)["items"]
+    split = {tuple(i["out_shape"]): "32x32x16_bf16" in i["source"] for i in items if i["class"] == "gemm_mfma_f32"}
+    kinds = [("32x32x16_bf16" in i["source"], i["out_shape"]) for i in items if i["class"] == "gemm_mfma_f32"]
+    assert kinds[0] == (False, [640, 700]), kinds  # z1, under relu
+    assert split[(640, 650)] and split[(700, 600)] and split[(650, 700)], kinds
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 def test_split_is_as_accurate_as_f32_sums(fg, hip, shape):
