@@ -465,8 +465,12 @@ class Emitter {
   // as a uniform byte offset `coef * size * kvar` in the scalar offset. The
   // caller renders `k` as its per-lane part only (the k-tile's start is
   // `kvar`), and every index must be affine with non-negative terms.
-  void set_buffer_loads(std::map<const UOpInner*, std::string> rsrc, const UOp& k, const std::string& kvar) {
+  // With `dwords`, four lanes along k load 16 bytes from any element: a buffer
+  // load needs the alignment of its 4-byte elements only.
+  void set_buffer_loads(std::map<const UOpInner*, std::string> rsrc, const UOp& k, const std::string& kvar,
+                        bool dwords = false) {
     buf_rsrc_ = std::move(rsrc);
+    buf_dwords_ = dwords;
     buf_k_ = k;
     buf_kvar_ = kvar;
   }
@@ -519,7 +523,7 @@ class Emitter {
         FG_CHECK(esz == 4, "buffer loads read 4-byte elements");
         const std::string soff = "(unsigned)(" + std::to_string(a.coef(buf_k_) * esz) + " * " + buf_kvar_ + ")";
         const bool f32 = n.dtype().kind == DTypeKind::F32;
-        if (lane_dep && vec4_load(n)) {
+        if (lane_dep && (vec4_load(n) || (lanes_ == 4 && buf_dwords_ && a.coef(buf_k_) == 1 && buf_k_.get() == lane_range_))) {
           std::string v = fresh("vec");
           const char* vt = f32 ? "fg_f4" : "fg_i4";
           emit_at(si, std::string("const ") + vt + " " + v + " = __builtin_bit_cast(" + vt +
@@ -611,6 +615,7 @@ class Emitter {
   std::map<const UOpInner*, std::string> buf_rsrc_;
   UOp buf_k_;
   std::string buf_kvar_;
+  bool buf_dwords_ = false;
   static bool is_index_expr(const UOp& n) {
     if (n.op() == Op::Range || n.op() == Op::Const || n.op() == Op::ParamScalar) return true;
     if (n.op() == Op::Add || n.op() == Op::Mul) return is_index_expr(n.src(0)) && is_index_expr(n.src(1));
@@ -3458,7 +3463,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       em.define_range(op.rout, "(long)grc");
       if (loads && bufl) {
         em.define_range(g.rk, "(long)kk");
-        em.set_buffer_loads(rsrc, g.rk, "k0c");
+        em.set_buffer_loads(rsrc, g.rk, "k0c", true);
       } else {
         em.define_range(g.rk, "(long)(k0c + kk)");
       }
