@@ -32,6 +32,22 @@ def test_split_row_reductions(fg, hip, shape, axes, narrowed):
     assert np.array_equal(got, i.sum(tuple(axes), keepdims=True, dtype=np.int32))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(60000, 17), (5000, 784), (3001, 66), (70000, 4), (9000, 1), (20, 3000, 18), (4097, 500)])
+def test_split_column_reductions(fg, hip, shape):
+    """Sums over the rows, split in chunks: ragged outputs of the second pass."""
+    a = np.random.default_rng(len(shape) + shape[-1]).standard_normal(shape).astype(np.float32)
+    axis = len(shape) - 2
+    x = fg.Tensor.new(a, list(shape), hip)
+    got = x.mul(x).sum([axis]).add(fg.Tensor.scalar(1.0, hip)).numpy()
+    want = (a.astype(np.float64) ** 2).sum(axis, keepdims=True) + 1.0
+    # At most 1100 rows of a thread's share and 40 more additions: 2^-24 each.
+    assert np.max(np.abs(got - want) / want) <= 1e-5
+    assert np.array_equal(x.max([axis]).numpy(), a.max(axis, keepdims=True))
+    i = (a * 100).astype(np.int32)
+    assert np.array_equal(fg.Tensor.new(i, list(shape), hip).sum([axis]).numpy(), i.sum(axis, keepdims=True, dtype=np.int32))
+
+
 def test_split_row_reduction_launches(fg, cpu):
     """[5000, 3001] summed whole: one merged range, several chunks."""
     x = fg.Tensor.zeros([5000, 3001], cpu).add(fg.Tensor.scalar(1.0, cpu))
