@@ -8,7 +8,8 @@ lowering-cache lookup, launch) with the inputs resident in HBM.
 
 Also measured and reported under "secondary": C1 (fused elementwise + row
 reduction, GB/s), C3 (Linear forward x@W^T+b, MFMA fp32 TFLOP/s), C4 and C5
-(MLP train steps/s plus the GEMM kernels' share of the fp32 MFMA peak).
+(MLP train steps/s plus the GEMM kernels' share of the fp32 MFMA peak; products
+split for the bfloat16 matrix cores can pass it).
 
 Kernel durations come from HIP events recorded around every launch on the
 device's own stream during the timed region (fg_hip_profile_*). The CPU
@@ -33,6 +34,8 @@ sys.path.insert(0, ROOT)
 METRIC = "fused-kernel HBM GB/s & MFMA fp32 TFLOP/s; MLP train steps/s (1 GPU)"
 HBM_PEAK_GBS = 8000.0           # MI355X HBM3E
 FP32_MFMA_PEAK_TFLOPS = 157.3   # MI355X dense fp32 matrix
+# An f32 product split into six bfloat16 products (C3's GEMM): a sixth of the dense bfloat16 matrix peak.
+SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 6
 
 
 def log(*a):
@@ -241,8 +244,8 @@ def bench_c3(fg, ctx, steps, warmup):
     check = {"against": "float64, 64 sampled rows", "max_err_over_bound": worst, "ok": worst <= 1.0}
     return {"ms_per_step": ms, "tflops_step": flops / (ms / 1e3) / 1e12, "kernels": kern, "check": check,
             "host_ms_per_step": timed.host_ms,
-            "roofline": {"bound": "mfma", "achieved": tf, "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                         "frac": tf / FP32_MFMA_PEAK_TFLOPS, "kernel": gemm[0] if gemm else None,
+            "roofline": {"bound": "mfma", "achieved": tf, "peak": SPLIT_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
+                         "frac": tf / SPLIT_MFMA_PEAK_TFLOPS, "kernel": gemm[0] if gemm else None,
                          "traffic": pmc_traffic(gemm[0]) if gemm else None, "algorithmic_flops": flops,
                          "kernel_avg_ms": g["avg_ms"]}}
 
