@@ -93,10 +93,10 @@ struct RenderedKernel {
   // Kernels that compute `rows` rows of outputs (their outermost range)
   // independently: the device function of (parameters, first row, row count)
   // that a 256-thread workgroup runs, its source and parameter types, and per
-  // parameter the elements between the rows it accesses (0: none by row; -1:
-  // elements of other rows too), so a device can run several of them in one
-  // launch, a few rows per workgroup (render_row_batch). row_work: elements of
-  // a row, the most of its terms and outputs.
+  // parameter the elements between the rows it accesses (0: nothing that moves
+  // with the row; -1: elements of other rows too), so a device can run several
+  // of them in one launch, a few rows per workgroup (render_row_batch).
+  // row_work: elements of a row, the most of its terms and outputs.
   std::string row_fn, row_src;
   std::vector<std::string> row_types;
   std::vector<int64_t> row_stride;

@@ -996,10 +996,14 @@ void set_row_body(const KernelInfo& ki, const std::string& name, const std::stri
   rk->row_work = work;
   const UOp& r = ki.out_ranges[0];
   for (auto& [slot, p] : ki.params) {
+    // An access that does not move with the row (stride 0) reads an element of
+    // some row in every row: beside one by row it leaves the row.
     int64_t stride = 0;
+    bool accessed = false;
     auto use = [&](const UOp& index) {
       const int64_t s = row_stride_of(affine_of(index), r);
-      stride = stride == 0 ? s : s == 0 || s == stride ? stride : -1;
+      stride = !accessed || s == stride ? s : -1;
+      accessed = true;
     };
     if (p == ki.out_param) use(ki.out_index);
     for (auto& ld : loads_in(ki.value))

@@ -69,3 +69,77 @@ def test_kernels_that_read_other_rows_stay_apart(fg, cpu):
     z, t = cross_entropy(fg, cpu, (500, 300), 4)
     loss = z.cross_entropy(t)
     assert fg.debug_plan([loss.gradient([z])[0]], fuse=True, render_hip=True)["row_batches"] == []
+
+
+# Programs whose second kernel reads the first one's output both in its own row
+# and in every row (or the first one reads so what the second one writes): the
+# result of (fg, device, a [n, k], m [n, n]) and the float64 value.
+def outer_sum(fg, dev, a, m):
+    n = len(a)
+    d = fg.Tensor.new(a, list(a.shape), dev)
+    d = d.mul(d).sum([1])
+    d64 = (a.astype(np.float64) ** 2).sum(1, keepdims=True)
+    return d.expand([n, n]).add(d.permute([1, 0]).expand([n, n])), d64 + d64.T
+
+
+def normalised_adjacency(fg, dev, a, m):
+    n = len(a)
+    t = fg.Tensor.new(m, [n, n], dev)
+    d = t.sum([1]).reciprocal()
+    d64 = 1.0 / m.astype(np.float64).sum(1, keepdims=True)
+    return t.mul(d.expand([n, n])).mul(d.permute([1, 0]).expand([n, n])), m * d64 * d64.T
+
+
+def first_row_added(fg, dev, a, m):
+    x = fg.Tensor.new(m, list(m.shape), dev)
+    e = x.exp().contiguous()
+    e64 = np.exp(m.astype(np.float64))
+    return e.add(e.narrow(0, 0, 1).expand(list(m.shape))), e64 + e64[:1]
+
+
+MIXED = {f.__name__: f for f in (outer_sum, normalised_adjacency, first_row_added)}
+
+
+def mixed_inputs(n):
+    r = np.random.default_rng(n)
+    return r.uniform(0.5, 1.5, (n, 300)).astype(np.float32), r.uniform(0.5, 1.5, (n, n)).astype(np.float32)
+
+
+def together(plan):
+    """The pairs of plan items that share a row batch."""
+    runs = [range(b["first"], b["first"] + b["count"]) for b in plan["row_batches"]]
+    return {(i, j) for r in runs for i in r for j in r if i < j}
+
+
+@pytest.mark.parametrize("name", MIXED)
+def test_reads_by_row_and_of_every_row_stay_apart(fg, cpu, name):
+    """A buffer read in the kernel's own row and without the row is not by row."""
+    out, _ = MIXED[name](fg, cpu, *mixed_inputs(1024))
+    plan = fg.debug_plan([out], fuse=True, render_hip=True)
+    assert len(plan["items"]) == 2 and together(plan) == set(), plan["row_batches"]
+
+
+def test_every_row_read_before_an_update_stays_apart(fg, cpu):
+    """y reads w[r] and all of w; the update of w in the same schedule is by row."""
+    n = 1024
+    w = fg.Tensor.new(np.ones((n, 1), np.float32), [n, 1], cpu)
+    y = w.expand([n, n]).add(w.permute([1, 0]).expand([n, n]))
+    w.assign(fg.Tensor.new(np.ones((n, 300), np.float32), [n, 300], cpu).sum([1]))
+    plan = fg.debug_plan([y, w], fuse=True, render_hip=True)
+    assert len(plan["items"]) == 2 and together(plan) == set(), plan["row_batches"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", MIXED)
+@pytest.mark.parametrize("n", [1024, 2050])
+def test_replays_of_mixed_reads(fg, hip, name, n):
+    fg.clear_caches()
+    a, m = mixed_inputs(n)
+    first = None
+    for _ in range(4):
+        out, want = MIXED[name](fg, hip, a, m)
+        got = out.numpy()
+        # At most 300 or n positive terms, 2^-24 each, and a few roundings.
+        assert np.max(np.abs(got - want) / want) <= 2e-4
+        assert first is None or np.array_equal(got, first)
+        first = got.copy()
