@@ -1725,7 +1725,10 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   rk.source = std::string(kPrelude) + signature(ki, name, 256) + " {\n" + em.code() + "}\n";
   rk.block[0] = 256;
   rk.grid[0] = static_cast<unsigned>(grid);
-  if (row_kernel(ki) && NOUT == ki.out_ext[0]) {
+  // Groups that are the rows: every other output range is shared (or of extent
+  // 1), and the rows are not. Extents alone do not tell: of [n, n] outputs the
+  // groups of a reduction broadcast over the rows are the n columns.
+  if (row_kernel(ki) && NOUT == ki.out_ext[0] && std::find(shared.begin(), shared.end(), ki.out_ranges[0]) == shared.end()) {
     Emitter er;
     emit(er, true);
     set_row_body(ki, name, er.code(), std::max(rt.terms, B), &rk);

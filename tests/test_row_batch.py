@@ -143,3 +143,52 @@ def test_replays_of_mixed_reads(fg, hip, name, n):
         assert np.max(np.abs(got - want) / want) <= 2e-4
         assert first is None or np.array_equal(got, first)
         first = got.copy()
+
+
+def column_sums_added(fg, dev, a, m):
+    """A reduction broadcast over the rows of square outputs: its kernel reads
+    what the first one writes."""
+    n = len(a)
+    e = fg.Tensor.new(m, [n, n], dev).exp()
+    s = fg.Tensor.new(a, list(a.shape), dev).sum([1])
+    out = e.add(s.permute([1, 0]).expand([n, n]))
+    e64 = np.exp(m.astype(np.float64))
+    return [e, out], [e64, e64 + a.astype(np.float64).sum(1)[None, :]]
+
+
+def exp_of_column_sums(fg, dev, a, m):
+    """The same kernel as the writer of what the second one reads by row."""
+    n = len(a)
+    s = fg.Tensor.new(a, list(a.shape), dev).mul(fg.Tensor.scalar(0.01, dev)).sum([1])
+    o = fg.Tensor.new(m, [n, n], dev).add(s.permute([1, 0]).expand([n, n]))
+    o64 = m + (a.astype(np.float64) * float(np.float32(0.01))).sum(1)[None, :]
+    return [o, o.exp()], [o64, np.exp(o64)]
+
+
+BROADCAST = {f.__name__: f for f in (column_sums_added, exp_of_column_sums)}
+
+
+@pytest.mark.parametrize("name", BROADCAST)
+def test_reductions_broadcast_over_the_rows_stay_apart(fg, cpu, name):
+    roots, _ = BROADCAST[name](fg, cpu, *mixed_inputs(1024))
+    plan = fg.debug_plan(roots, fuse=True, render_hip=True)
+    reduces = [i for i, it in enumerate(plan["items"]) if it["class"] == "row_reduce"]
+    assert len(plan["items"]) == 2 and len(reduces) == 1 and together(plan) == set(), plan["row_batches"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", BROADCAST)
+@pytest.mark.parametrize("n", [1024, 2050])
+def test_replays_of_reductions_broadcast_over_the_rows(fg, hip, name, n):
+    fg.clear_caches()
+    a, m = mixed_inputs(n)
+    first = None
+    for _ in range(4):
+        roots, want = BROADCAST[name](fg, hip, a, m)
+        fg.Tensor.realize_many(roots)
+        got = [t.numpy() for t in roots]
+        for g, w in zip(got, want):
+            # Sums of 300 positive terms (of about 3 before exp), 2^-24 each.
+            assert np.max(np.abs(g - w) / w) <= 1e-4
+        assert first is None or all(np.array_equal(x, y) for x, y in zip(got, first))
+        first = [g.copy() for g in got]
