@@ -961,6 +961,8 @@ std::vector<UOp> loads_in(const UOp& v) {
   return out;
 }
 
+constexpr int64_t kComputeUnits = 256;  // MI355X
+
 std::string block_params(const KernelInfo& ki, std::vector<std::string>* types, std::vector<std::string>* names);
 
 // ── Row kernels ─────────────────────────────────────────────────────────────
@@ -1519,25 +1521,72 @@ RenderedKernel render_row_reduce_split(const KernelInfo& ki, const RowSplit& sp,
 // A kernel whose reduction does not move with some output ranges (a softmax
 // gradient's row sum inside an elementwise expression) folds the same terms
 // again for every output along them: x / sum(x) over f32 [4096, 1000] took
-// 541 us. Here T threads fold each row once, then walk the row's outputs.
+// 541 us. Here T threads fold each group of outputs once, then walk them.
 // The fold is bound by HBM; the walk re-reads the row from L2. Same box:
-// 541 -> 11.3 us. From kRowOutputsMinTerms terms on: shorter folds keep one
-// or two threads an output (8192 rows of 10 run in the time of a launch).
+// 541 -> 11.3 us.
+//
+// Folding again for every output costs about a microsecond for 8 million
+// terms (they sit in the caches), a walk of consecutive outputs one for about
+// 700,000 of them. So outputs are walked from kRowOutputsMinTerms terms on:
+// shorter folds keep one or two threads an output (8192 rows of 10 run in the
+// time of a launch). Groups whose outputs lie apart (fewer than
+// kRowOutputsMinRun in a row: a reduction broadcast over the rows) are walked a
+// cache line per lane, 56,000 outputs a microsecond, from
+// kRowOutputsMinTermsStrided terms on: [4096, 4096] with column sums of 64
+// terms 163 us folded again, 299 walked; of 300 terms 2190 and 297; [4096, 64,
+// 4], a sum of 128 terms for each of the 64, 19.8 and 9.7.
 constexpr int64_t kRowOutputsMinTerms = 64;
+constexpr int64_t kRowOutputsMinTermsStrided = 128;
+constexpr int64_t kRowOutputsMinRun = 64;
 
-// The output ranges the reduction does not move with (empty: none).
-std::vector<UOp> row_output_ranges(const KernelInfo& ki) {
-  std::vector<UOp> out;
+struct RowOutputs {
+  std::vector<UOp> shared;  // the output ranges the reduction does not move with (empty: none)
+  int64_t B = 1;            // outputs of a group
+};
+
+RowOutputs row_outputs(const KernelInfo& ki) {
+  RowOutputs ro;
   const UOp& R = ki.reduces[0];
   UOpSet used;
   for (auto& n : R.toposort())
     if (n.op() == Op::Range) used.insert(n);
   int64_t terms = 1;
   for (size_t i = 1; i < R.srcs().size(); i++) terms *= range_extent(R.src(i));
-  if (terms < kRowOutputsMinTerms) return out;
-  for (size_t i = 0; i < ki.out_ranges.size(); i++)
-    if (!used.count(ki.out_ranges[i]) && ki.out_ext[i] > 1) out.push_back(ki.out_ranges[i]);
-  return out;
+  for (size_t i = 0; i < ki.out_ranges.size(); i++) {
+    if (used.count(ki.out_ranges[i]) || ki.out_ext[i] <= 1) continue;
+    ro.shared.push_back(ki.out_ranges[i]);
+    ro.B *= ki.out_ext[i];
+  }
+  // Consecutive outputs of a group: along the shared ranges that continue one another.
+  const Affine a = affine_of(ki.out_index);
+  int64_t run = 1;
+  for (bool more = a.ok; more;) {
+    more = false;
+    for (size_t i = 0; i < ki.out_ranges.size(); i++)
+      if (ki.out_ext[i] > 1 && a.coef(ki.out_ranges[i]) == run &&
+          std::find(ro.shared.begin(), ro.shared.end(), ki.out_ranges[i]) != ro.shared.end()) {
+        run *= ki.out_ext[i];
+        more = true;
+        break;
+      }
+  }
+  if (terms < (run < kRowOutputsMinRun ? kRowOutputsMinTermsStrided : kRowOutputsMinTerms)) ro = RowOutputs{};
+  return ro;
+}
+
+// Workgroups that walk one group's outputs, each folding the group's terms:
+// one where there is a group for each CU ([256, 65536] minus its row maxima:
+// 35.8 us, 39.9 with two). Fewer groups leave CUs idle ([4096, 4096] times the
+// sum of 256 terms has one group: 7151 us on one workgroup). They are cut to
+// about four workgroups per CU where the fold is short beside the walk (27.8 us
+// with two per CU, 23.2 with four, 24.7 with eight), else to one per CU and
+// to walks not much shorter than the fold: more only fold again, through the
+// shared caches ([64, 65536] 18.3 us with 4, 18.2 with 16; [64, 262144] 59.9
+// with 4, 99.8 with 16).
+int64_t row_output_cuts(int64_t groups, int64_t outputs, int64_t terms) {
+  if (groups >= kComputeUnits || terms == 0) return 1;
+  const int64_t want = outputs >= 16 * terms ? 4 * kComputeUnits : kComputeUnits;
+  return std::max<int64_t>(1, std::min({want / groups, outputs / 2048, 4 * outputs / terms}));
 }
 
 // ── RowReduce ───────────────────────────────────────────────────────────────
@@ -1550,18 +1599,17 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
   const UOp r_in = ranges.back();
   int64_t L = range_extent(r_in);
   // Outputs that share a reduction: NOUT groups (rows) of B.
-  const std::vector<UOp> shared = row_output_ranges(ki);
-  int64_t NOUT = total_outputs(ki), B = 1;
-  for (size_t i = 0; i < ki.out_ranges.size(); i++)
-    if (std::find(shared.begin(), shared.end(), ki.out_ranges[i]) != shared.end()) B *= ki.out_ext[i];
-  NOUT /= B;
+  const RowOutputs ro = row_outputs(ki);
+  const std::vector<UOp>& shared = ro.shared;
+  const int64_t B = ro.B, NOUT = total_outputs(ki) / B;
   int T = std::min<int>(256, pow2_floor(std::max<int64_t>(1, shared.empty() ? L / 16 : std::max(L, B) / 8)));
   int OPW = 256 / T;  // outputs (or rows of them) per workgroup
   // Vector width along r_in: all lane-dependent loads unit-stride and aligned.
   const int V = L % 4 == 0 && row_loads_vec4(rt.value, r_in) ? 4 : 1;
   RowSplit sp;
   if (L > 0 && shared.empty() && row_split(ki, rt, rt.terms / L * ((L + T * V - 1) / (T * V)), &sp)) return render_row_reduce_split(ki, sp, name);
-  const int64_t grid = (NOUT + OPW - 1) / OPW;
+  const int64_t cuts = !shared.empty() && OPW == 1 ? row_output_cuts(NOUT, B, rt.terms) : 1;
+  const int64_t grid = (NOUT + OPW - 1) / OPW * cuts;
   // The kernel, or with `rows` the body that computes rows [row0, row0 + nrows)
   // (one group of outputs each) on one workgroup.
   auto emit = [&](Emitter& em, bool rows) {
@@ -1592,7 +1640,7 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
     // interleaved order, which spreads the 8 XCDs' reads over HBM better.)
     em.line("const long bid = (long)(blockIdx.x % 8) * " + std::to_string(grid / 8) + " + blockIdx.x / 8;");
   } else {
-    em.line("const long bid = blockIdx.x;");
+    em.line("const long bid = blockIdx.x" + (cuts > 1 ? " / " + std::to_string(cuts) : std::string()) + ";");
   }
   if (!rows) {
     em.line("const long oid = bid * " + std::to_string(OPW) + " + tid / " + std::to_string(T) + ";");
@@ -1690,7 +1738,14 @@ RenderedKernel render_row_reduce(const KernelInfo& ki, const std::string& name) 
                   (odt.kind == DTypeKind::F32 || odt.kind == DTypeKind::I32);
     for (auto& t : ao.terms)
       if (t.first != fast && t.second % 4 != 0) vstore = false;
-    em.open_scope("if (active) for (int b = rlane; b < " + std::to_string(B / VB) + "; b += " + std::to_string(T) + ") {", "}");
+    std::string b0 = "rlane", b1 = std::to_string(B / VB);
+    if (cuts > 1 && !rows) {
+      const std::string per = std::to_string((B / VB + cuts - 1) / cuts);
+      em.line("const int cut = (int)(blockIdx.x % " + std::to_string(cuts) + ") * " + per + ";");
+      b0 = "cut + rlane";
+      b1 = "(cut + " + per + " < " + b1 + " ? cut + " + per + " : " + b1 + ")";
+    }
+    em.open_scope("if (active) for (int b = " + b0 + "; b < " + b1 + "; b += " + std::to_string(T) + ") {", "}");
     // The fast range innermost, the others in output order.
     std::string rest = "b";
     auto take = [&](const UOp& r, int64_t e, int V) {
@@ -2063,7 +2118,6 @@ std::vector<KmChunk> km_chunks(int T) {
   return out;
 }
 
-constexpr int64_t kComputeUnits = 256;  // MI355X
 constexpr int kGemmStageK = 16;         // k of one LDS stage of the tiled GEMM, one MFMA deep
 constexpr int kGemmFoldTiles = 5;       // 32x32 tiles of a wave up to which every 2nd stage is folded apart, else every 4th
 constexpr int64_t kLdsPerCu = 163840;   // gfx950 LDS bytes per CU
