@@ -3775,7 +3775,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     for (int j = 0; j < EW / 32; j++) {
       floatx16 t = acc[i][jj * (EW / 32) + j];
       #pragma unroll
-      for (int e = 0; e < 16; e++) t[e] *= e & 1 ? -descale : descale;
+      for (int e = 0; e < 16; e++) t[e] = t[e] * (e & 1 ? -descale : descale) + 0.0f;  // a zero sum is +0
       if (again) t = f32_tile(i, jj * (EW / 32) + j);
       #pragma unroll
       for (int e = 0; e < 16; e++) wst[(8 * (e >> 2) + 4 * h + (e & 3)) * EPS + 32 * j + r32] = t[e];

@@ -80,3 +80,15 @@ def test_infinities_nan_and_overflow(fg, hip, shape):
         assert np.array_equal(got[over & np.isinf(want)], want[over & np.isinf(want)]), name
         fine = ~np.isnan(want) & ~over & (terms < 3.3e38)
         assert np.all(np.abs(got[fine] - want[fine]) <= 1e-5 * terms[fine]), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_zero_sums_are_positive(fg, hip, shape):
+    """Zero rows and zero columns of operands (a dead unit, a padded batch)
+    give +0 wherever they fall in a tile, as sums that start from +0 do."""
+    x, w, g = data(shape, 4)
+    x[::3], x[:, ::7], w[::5], g[1::4], g[:, 2::6] = 0.0, 0.0, 0.0, 0.0, 0.0
+    for name, (got, want, terms) in run(fg, hip, x, w, g).items():
+        assert np.any(terms == 0), name
+        assert np.all(got[terms == 0] == 0) and not np.any(np.signbit(got[terms == 0])), name
