@@ -2119,7 +2119,11 @@ std::vector<KmChunk> km_chunks(int T) {
 }
 
 constexpr int kGemmStageK = 16;         // k of one LDS stage of the tiled GEMM, one MFMA deep
-constexpr int kGemmFoldTiles = 5;       // 32x32 tiles of a wave up to which every 2nd stage is folded apart, else every 4th
+// Stages whose products are summed apart (see render_gemm): every one up to K
+// kGemmFoldAllK; every 2nd up to kGemmFold2K and for waves of at most
+// kGemmFoldTiles tiles of 32x32; else every 4th.
+constexpr int64_t kGemmFoldAllK = 1024, kGemmFold2K = 2048;
+constexpr int kGemmFoldTiles = 5;
 constexpr int64_t kLdsPerCu = 163840;   // gfx950 LDS bytes per CU
 constexpr int64_t kMinSplitK = 64;      // shortest K range a split workgroup runs
 
@@ -3371,8 +3375,14 @@ RenderedKernel render_gemm_f32(const KernelInfo& ki, const GemmMatch& g, const s
 // operands in memory.
 //
 // Error against 64 bits (2-norm): the six products are added to the running
-// sums one after another, smallest first, except in every 2nd stage (waves of
-// few tiles) or 4th, whose products are summed apart and added once. The
+// sums one after another, smallest first, except in the stages whose products
+// are summed apart and added once: every 4th, every 2nd for waves of few tiles
+// and up to a K of 2048, and every one up to 1024, where the f32 tiles keep
+// their chains short by splitting K. With every 2nd, 1030x1010 of K 320 had an
+// error of 2.06e-7 (positive operands 1.62e-7), now 9.9e-8 (6.9e-8); the f32
+// tiles 1.51e-7 (6.7e-8). It costs 0-5% there (4096x1024 of K 784 53.1 -> 55.3
+// us), 25% at 3000x1500 of K 1500. Of 50 products of 33 to 4096 k none is above
+// the f32 tiles, of positive operands a few (by up to 9%). The
 // bfloat16 MFMA rounds the aligned sum down, so the operands' odd rows are
 // negated and the results' signs alternate: without that the errors of all
 // sums leaned the same way (mean -2.1e-7 of their spread at K 4096, 1e-10
@@ -3386,7 +3396,7 @@ RenderedKernel render_gemm_f32(const KernelInfo& ki, const GemmMatch& g, const s
 // register-only bfloat16 MFMAs on the same data at 267-310. Loads two stages
 // ahead, wave priorities, 4 waves of 128x128 (196-200) and sched_group_barrier
 // interleaving did not help. Summing every stage's products apart (error
-// 3.1e-7) cost 9-11%, every 4th 0-4%.
+// 3.1e-7) cost 9-11% at this K, every 4th 0-4%.
 RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::string& name) {
   if (small_gemm_fits(g.M, g.N, g.K)) return render_small_gemm(ki, g, name);
   if (ki.compared || gemm_hbm_bound(g.M, g.N, g.K)) return render_gemm_f32(ki, g, name);
@@ -3444,7 +3454,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
   s << "#define S_ " << S << "\n#define KC_ " << KC << "\n#define NTILES_ " << ntiles << "\n";
   s << "#define BM " << BM << "\n#define BN " << BN << "\n#define BK " << BK << "\n";
   s << "#define NT " << NT << "\n#define WGN " << WGN << "\n#define TM " << TM << "\n#define TN " << TN << "\n";
-  s << "#define NBUF_ " << tile.nbuf << "\n#define FOLD_ " << (TM * TN <= kGemmFoldTiles ? 2 : 4) << "\n";
+  s << "#define NBUF_ " << tile.nbuf << "\n#define FOLD_ " << (K <= kGemmFoldAllK ? 1 : K <= kGemmFold2K || TM * TN <= kGemmFoldTiles ? 2 : 4) << "\n";
   if (tile.stream_k) {
     s << "#define G_ " << tile.G << "\n#define KTT_ " << KTT << "\n#define ITERS_ " << ntiles * KTT << "L\n";
     if (sk_D > 0) s << "#define SK_D_ " << sk_D << "\n";

@@ -92,3 +92,39 @@ def test_zero_sums_are_positive(fg, hip, shape):
     for name, (got, want, terms) in run(fg, hip, x, w, g).items():
         assert np.any(terms == 0), name
         assert np.all(got[terms == 0] == 0) and not np.any(np.signbit(got[terms == 0])), name
+
+
+# (B, in, out) whose forward product has K from 100 to 1030, where chains of
+# f32 sums are short; errors of the f32 tiles' sums of the same products, of
+# normal and of positive operands (2-norm, measured). From K 1024 on, where
+# every 2nd stage is folded, sums of positive operands may be a tenth above
+# (K 1030: 2.62e-7, the f32 tiles' 2.45e-7).
+SHORT = [((1030, 100, 1010), 1.8e-7, 1.4e-7), ((1030, 256, 1010), 2.0e-7, 1.3e-7), ((1030, 320, 1010), 1.5e-7, 7.5e-8),
+         ((1030, 512, 1010), 1.65e-7, 7.1e-8), ((4096, 784, 1024), 3.5e-7, 1.95e-7), ((4096, 1030, 1024), 4.0e-7, 2.7e-7)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,normal,positive", SHORT)
+def test_short_products_are_as_accurate_as_f32_sums(fg, hip, shape, normal, positive):
+    x, w, _ = data(shape, 5)
+    for a, b, bound in ((x, w, normal), (np.abs(x), np.abs(w), positive)):
+        t = fg.Tensor.new(a, list(a.shape), hip).matmul(fg.Tensor.new(b, list(b.shape), hip).permute([1, 0]))
+        want = a.astype(np.float64) @ b.astype(np.float64).T
+        got = t.numpy().reshape(want.shape)
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= bound
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,normal,positive", SHORT)
+def test_cancelling_sums(fg, hip, shape, normal, positive):
+    """Products whose second half of k cancels the first: an error within the
+    rounding of the terms' own sums, for each element."""
+    x, w, _ = data(shape, 6)
+    h = shape[1] // 2
+    x[:, h:2 * h] = -x[:, :h]
+    w[:, h:2 * h] = w[:, :h] * (1.0 + 1e-3 * np.random.default_rng(7).standard_normal((len(w), h)).astype(np.float32))
+    t = fg.Tensor.new(x, list(x.shape), hip).matmul(fg.Tensor.new(w, list(w.shape), hip).permute([1, 0]))
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    terms = np.abs(x64) @ np.abs(w64).T
+    # The largest of the f32 tiles' sums is 2.7e-7 of the terms (K 128).
+    assert np.max(np.abs(t.numpy().reshape(terms.shape) - x64 @ w64.T) / terms) <= 2.7e-7
