@@ -1025,7 +1025,7 @@ bool row_kernel(const KernelInfo& ki) {
 // (a permuted copy, an operand read through a transpose) costs the plain
 // elementwise kernel a cache line per lane: a transposed copy of f32
 // [4000, 3001] ran at 1.5 TB/s (64.8 us), one of [33000, 508] at 0.6. Here a
-// workgroup takes a tile of kTileElems outputs, reads the tile along the
+// workgroup takes a tile of up to kTileElems outputs, reads the tile along the
 // load's own unit stride into LDS and computes and stores it along the
 // stores'. Both sides then move whole 256-byte runs. LDS rows have an odd
 // pitch, so reading a column is free of bank conflicts. Same box: 64.8 -> 19.2
@@ -1033,11 +1033,18 @@ bool row_kernel(const KernelInfo& ki) {
 // (5.3 TB/s).
 constexpr int64_t kTileElems = 4096;
 constexpr int kTileThreads = 256;
-constexpr size_t kTileMaxLoads = 3;  // 16.6 KB of LDS each
+constexpr size_t kTileMaxLoads = 3;  // 16.6 KB of LDS each, up to 24.6 where a side of 2 is padded to 3
 // Outputs from which the tiles are used. Below, the operands sit in L2 and
 // both kernels take little more than their launch (2^20: 4.4-6.8 us plain, 4.4-4.9 tiled; 2^16:
 // 4.0 either way).
 constexpr int64_t kTileMinOutputs = int64_t(1) << 18;
+// Outputs of a tile from which the tiles are used: a tile lies in one pair of
+// the two ranges, so many small transposes have small tiles, whose cache lines
+// the plain kernel's lanes share anyway. Plain and tiled, us a call: 262144 of
+// 2 x 2 6.6 and 63, 65536 of 8 x 8 7.1 and 17, 65536 of 16 x 16 20.3 and 22.0,
+// 32768 of 4 x 64 11.2 and 12.4; 20000 of 10 x 40 21.7 and 12.7, of 40 x 10 14.8
+// and 11.6; 30000 of 31 x 17 49.7 and 22.1.
+constexpr int64_t kTileMinElems = 384;
 
 struct TilePlan {
   UOp f, g;                // unit-stride ranges of the store and of the staged loads
@@ -1072,11 +1079,11 @@ bool tile_plan(const KernelInfo& ki, TilePlan* tp) {
   tp->F = extent(f);
   tp->G = extent(tp->g);
   if (tp->F < 2 || tp->G < 2) return false;
-  // 64 x 64, or all of a side shorter than that by more of the other.
+  // 64 x 64, or all of a side shorter than that by more (up to all) of the other.
   auto rest = [](int64_t side) { return std::max<int64_t>(64, kTileElems / side / 64 * 64); };
-  tp->TF = tp->F < 64 ? tp->F : tp->G < 64 ? rest(tp->G) : 64;
-  tp->TG = tp->F < 64 ? rest(tp->F) : std::min<int64_t>(64, tp->G);
-  return true;
+  tp->TF = std::min(tp->F, tp->F >= 64 && tp->G < 64 ? rest(tp->G) : 64);
+  tp->TG = std::min(tp->G, tp->F < 64 ? rest(tp->F) : 64);
+  return tp->TF * tp->TG >= kTileMinElems;
 }
 
 RenderedKernel render_elementwise_tiled(const KernelInfo& ki, const TilePlan& tp, const std::string& name) {
