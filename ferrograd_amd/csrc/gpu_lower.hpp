@@ -188,8 +188,9 @@ std::vector<size_t> pair_runs(const std::vector<const RenderedKernel*>& kernels,
 RenderedKernel render_row_batch(const std::vector<const RenderedKernel*>& stages);
 // The runs of two or more consecutive row kernels that can share such a
 // launch, as (first, count) pairs: same row count, none marked in `excluded`,
-// at most kMaxBatchStages kernels and FG_MAX_LAUNCH_ARGS arguments, and every
-// buffer one of them writes accessed by the others only in the same rows.
+// at most kMaxBatchStages kernels and FG_MAX_LAUNCH_ARGS arguments, every
+// buffer one of them writes accessed by the others only in the same rows, and
+// rows or operands that stay in the caches.
 std::vector<std::pair<size_t, size_t>> row_batch_runs(const std::vector<const RenderedKernel*>& kernels,
                                                       const std::vector<std::vector<BatchArg>>& args,
                                                       const std::vector<bool>& excluded);

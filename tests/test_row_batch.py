@@ -192,3 +192,16 @@ def test_replays_of_reductions_broadcast_over_the_rows(fg, hip, name, n):
             assert np.max(np.abs(g - w) / w) <= 1e-4
         assert first is None or all(np.array_equal(x, y) for x, y in zip(got, first))
         first = [g.copy() for g in got]
+
+
+def test_long_rows_batch_while_they_stay_in_the_caches(fg, cpu):
+    def runs(rows, cols):
+        x = fg.Tensor.zeros([rows, cols], cpu).add(fg.Tensor.scalar(1.0, cpu)).realize()
+        e = x.exp()
+        plan = fg.debug_plan([e, e.mul(x)], fuse=True, render_hip=True)
+        assert len(plan["items"]) == 2
+        return [(b["first"], b["count"]) for b in plan["row_batches"]]
+
+    # Three buffers of rows x cols: up to 8192 columns, or 256 MiB in all.
+    assert runs(4096, 8192) == [(0, 2)] and runs(600, 32768) == [(0, 2)]
+    assert runs(1024, 32768) == [] and runs(512, 131072) == [] and runs(4096, 8196) == []
