@@ -3379,7 +3379,8 @@ RenderedKernel render_gemm_f32(const KernelInfo& ki, const GemmMatch& g, const s
 // has parts that are exact in bfloat16, and the sums (scaled by 2^32) are
 // scaled back in the epilogue. A tile whose sums are not finite (infinities,
 // NaN, |sum| of 2^96 and more) is computed again with the f32 MFMA from the
-// operands in memory.
+// operands in memory: 4096^3 with such a sum in every tile 1.5 ms, 0.7 without
+// one (7.7 with loads of every element by itself; the f32 tiles 1.0 either way).
 //
 // Error against 64 bits (2-norm): the six products are added to the running
 // sums one after another, smallest first, except in the stages whose products
@@ -3593,7 +3594,9 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       l << indent(em.code() + body.str(), "      ");
     }
     l << "    }\n  };\n";
-    l << "  auto store_" << X << " = [&](fg_raw& w, int buf, int k0) {\n" << k0c;
+    // store_X writes the parts, store_f32_X the values as they are.
+    for (const bool parts : {true, false}) {
+    l << "  auto store_" << (parts ? "" : "f32_") << X << " = [&](fg_raw& w, int buf, int k0) {\n" << k0c;
     l << "    #pragma unroll\n    for (int j = 0; j < " << st.per << "; j++) {\n" << coords;
     {
       Emitter em;
@@ -3611,9 +3614,11 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
         std::string in;
         if (k_ragged) in = "k0c + " + k + " >= k0";
         if (k_inner) in += (in.empty() ? "" : " && ") + std::string("k0c + ") + k + " < kend";
-        body << "v[" << u << "] = " << vals[u] << " * " << (in.empty() ? "sc" : "(" + in + " ? sc : 0.0f)") << ";\n";
+        if (parts) body << "v[" << u << "] = " << vals[u] << " * " << (in.empty() ? "sc" : "(" + in + " ? sc : 0.0f)") << ";\n";
+        else body << "v[" << u << "] = " << (in.empty() ? vals[u] : in + " ? " + vals[u] + " : 0.0f") << ";\n";
       }
-      l << "      const float sc = (r & 1) ? -65536.0f : 65536.0f;\n      float v[" << V << "];\n";
+      if (parts) l << "      const float sc = (r & 1) ? -65536.0f : 65536.0f;\n";
+      l << "      float v[" << V << "];\n";
       if (!(st.lds.size() == 1 && op.expr == st.lds[0])) {
         // The operand is an expression of its loads (a relu recomputed, a
         // mask): pass the raw registers through an empty asm here, so the
@@ -3627,21 +3632,21 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       l << indent(em.code() + body.str(), "      ");
     }
     const std::string PL = X[0] == 'a' ? "PLA" : "PLB";
-    l << "      char* at = smem + buf * STG + " << (X[0] == 'a' ? "0" : "6 * PLA") << " + (kk >> 3) * " << PL << " + r * 16"
-      << (st.k_fast ? " + (kk & 4) * 2" : "") << ";\n";
-    l << "      int p[3][" << V / 2 << "];\n";
-    l << "      #pragma unroll\n      for (int u = 0; u < " << V / 2
-      << "; u++) fg_split(v[2 * u], v[2 * u + 1], p[0][u], p[1][u], p[2][u]);\n";
-    l << "      #pragma unroll\n      for (int q = 0; q < 3; q++) ";
-    if (st.k_fast) l << "*(fg_i2*)(at + 2 * q * " << PL << ") = fg_i2{p[q][0], p[q][1]};\n";
-    else l << "*(fg_i4*)(at + 2 * q * " << PL << ") = fg_i4{p[q][0], p[q][1], p[q][2], p[q][3]};\n";
+    l << "      char* at = smem + buf * STG + " << (X[0] == 'a' ? "0" : "6 * PLA") << " + (kk >> " << (parts ? 3 : 2) << ") * " << PL
+      << " + r * 16" << (parts && st.k_fast ? " + (kk & 4) * 2" : "") << ";\n";
+    if (parts) {
+      l << "      int p[3][" << V / 2 << "];\n";
+      l << "      #pragma unroll\n      for (int u = 0; u < " << V / 2
+        << "; u++) fg_split(v[2 * u], v[2 * u + 1], p[0][u], p[1][u], p[2][u]);\n";
+      l << "      #pragma unroll\n      for (int q = 0; q < 3; q++) ";
+      if (st.k_fast) l << "*(fg_i2*)(at + 2 * q * " << PL << ") = fg_i2{p[q][0], p[q][1]};\n";
+      else l << "*(fg_i4*)(at + 2 * q * " << PL << ") = fg_i4{p[q][0], p[q][1], p[q][2], p[q][3]};\n";
+    } else {
+      l << "      #pragma unroll\n      for (int q = 0; q < " << V / 4 << "; q++) *(fg_f4*)(at + q * " << PL
+        << ") = fg_f4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};\n";
+    }
     l << "    }\n  };\n";
-    // One element of the operand at row gr and k gk, in f32.
-    Emitter em;
-    em.define_range(op.rout, "(long)gr");
-    em.define_range(g.rk, "(long)gk");
-    const std::string v = em.val(op.expr, 0);
-    l << "  auto at_" << X << " = [&](int gr, int gk) {\n" << indent(em.code(), "  ") << "    return " << v << ";\n  };\n";
+    }
     return l.str();
   };
   s << loader("a", g.a, sa, BM, M, "m");
@@ -3752,8 +3757,10 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
 #endif
   #pragma unroll 1
   for (; kt < KT; kt++) stage(FOLD_ == 1, kt);
-  // Sums that are not finite (infinite operands, overflow of the scaled sums)
-  // are computed again from the f32 operands, one 32x32 tile at a time.
+  // Where a sum is not finite (operands that are not, overflow of the scaled
+  // sums), the workgroup computes its tile again with the f32 MFMA: stages of
+  // 16 k as [4 k][row] chunks of 16 bytes in the parts' planes, two in turn
+  // (the barrier after one is written ends the reads of the one before).
   float chk = 0.0f;
   #pragma unroll
   for (int i = 0; i < TM; i++)
@@ -3764,22 +3771,39 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
   if (chk != chk) fg_bad = 1;
   __syncthreads();
   const bool again = fg_bad != 0;
-  const float descale = r32 & 1 ? -0x1p-32f : 0x1p-32f;  // row and column signs
-  auto f32_tile = [&](int i, int j) {
-    const int ra = m0 + wm + 32 * i + r32, rb = n0 + wn + 32 * j + r32;
-    const int rac = ra < M_ ? ra : M_ - 1, rbc = rb < N_ ? rb : N_ - 1;
-    floatx16 t;
+  // Selected rather than branched around, so the sums stay in their registers.
+  #pragma unroll
+  for (int i = 0; i < TM; i++)
     #pragma unroll
-    for (int e = 0; e < 16; e++) t[e] = 0.0f;
-    #pragma unroll 1
-    for (int k = kbeg; k < kend; k += 2) {
-      const bool in = k + h < kend;
-      const int gk = in ? k + h : k;
-      const float va = at_a(rac, gk), vb = at_b(rbc, gk);
-      t = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? va : 0.0f, in ? vb : 0.0f, t, 0, 0, 0);
+    for (int j = 0; j < TN; j++)
+      #pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] = again ? 0.0f : acc[i][j][e];
+  if (again) { load_a(w, kat(0)); load_b(w, kat(0)); }
+  const int redo = again ? KT : 0;
+  #pragma unroll 1
+  for (int t = 0; t < redo; t++) {
+    store_f32_a(w, t & 1, kat(t)); store_f32_b(w, t & 1, kat(t));
+    load_a(w, kat(t + 1)); load_b(w, kat(t + 1));
+    __syncthreads();
+    const char* at = smem + (t & 1) * STG;
+    #pragma unroll
+    for (int q = 0; q < 2; q++) {  // of the 8 k of q, the lane half's 4
+      fg_f4 va[TM], vb[TN];
+      #pragma unroll
+      for (int i = 0; i < TM; i++) va[i] = *(const fg_f4*)(at + (2 * q + h) * PLA + (wm + 32 * i + r32) * 16);
+      #pragma unroll
+      for (int j = 0; j < TN; j++) vb[j] = *(const fg_f4*)(at + 6 * PLA + (2 * q + h) * PLB + (wn + 32 * j + r32) * 16);
+      #pragma unroll
+      for (int u = 0; u < 4; u++)
+        #pragma unroll
+        for (int i = 0; i < TM; i++)
+          #pragma unroll
+          for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[i][u], vb[j][u], acc[i][j], 0, 0, 0);
     }
-    return t;
-  };
+  }
+  __syncthreads();
+  // What scales a lane's even and odd rows back, row and column signs included.
+  const float even = again ? 1.0f : r32 & 1 ? -0x1p-32f : 0x1p-32f, odd = again ? 1.0f : -even;
   // Epilogue: each wave stages 32 x EW accumulators in its own LDS tile (32x32
   // MFMA layout: element e of lane l is row 8*(e/4) + 4*(l/32) + e%4, column
   // l%32 of its tile), then reads them back as rows of float4, so epilogue
@@ -3792,8 +3816,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
     for (int j = 0; j < EW / 32; j++) {
       floatx16 t = acc[i][jj * (EW / 32) + j];
       #pragma unroll
-      for (int e = 0; e < 16; e++) t[e] = t[e] * (e & 1 ? -descale : descale) + 0.0f;  // a zero sum is +0
-      if (again) t = f32_tile(i, jj * (EW / 32) + j);
+      for (int e = 0; e < 16; e++) t[e] = t[e] * (e & 1 ? odd : even) + 0.0f;  // a zero sum is +0
       #pragma unroll
       for (int e = 0; e < 16; e++) wst[(8 * (e >> 2) + 4 * h + (e & 3)) * EPS + 32 * j + r32] = t[e];
     }

@@ -66,20 +66,34 @@ def test_operands_of_any_magnitude(fg, hip, shape):
         assert np.all(np.abs(got - want) <= bound), name
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("shape", SHAPES)
-def test_infinities_nan_and_overflow(fg, hip, shape):
+def check_not_finite(fg, dev, shape, big=3.4e38):
     x, w, g = data(shape, 3)
     x[5, 7], x[9, 3], x[11, 2] = np.inf, np.nan, -np.inf
-    w[2, 2], w[40, 40] = np.inf, 3.4e38
+    w[2, 2], w[40, 40] = np.inf, big
     x[300:303] *= np.float32(1e33)  # finite sums of 1e34 and more
-    g[4, 4], g[6, 100] = np.inf, 3.4e38
-    for name, (got, want, terms) in run(fg, hip, x, w, g).items():
+    g[4, 4], g[6, 100] = np.inf, big
+    for name, (got, want, terms) in run(fg, dev, x, w, g).items():
         assert np.array_equal(np.isnan(got), np.isnan(want)), name
         over = ~np.isnan(want) & (np.abs(want) > 3.3e38)
         assert np.array_equal(got[over & np.isinf(want)], want[over & np.isinf(want)]), name
         fine = ~np.isnan(want) & ~over & (terms < 3.3e38)
         assert np.all(np.abs(got[fine] - want[fine]) <= 1e-5 * terms[fine]), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_infinities_nan_and_overflow(fg, hip, shape):
+    check_not_finite(fg, hip, shape)
+
+
+# The largest finite value without products beyond f32: one of those beside an
+# infinity of the other sign is NaN in f32, but not in float64.
+BIG = 5e37
+
+
+@pytest.mark.gpu
+def test_infinities_nan_and_overflow_of_larger_products(fg, hip):
+    check_not_finite(fg, hip, (2050, 1030, 1000), BIG)
 
 
 @pytest.mark.gpu
@@ -128,3 +142,56 @@ def test_cancelling_sums(fg, hip, shape, normal, positive):
     terms = np.abs(x64) @ np.abs(w64).T
     # The largest of the f32 tiles' sums is 2.7e-7 of the terms (K 128).
     assert np.max(np.abs(t.numpy().reshape(terms.shape) - x64 @ w64.T) / terms) <= 2.7e-7
+
+
+# The same with the tile fixed, in a process of its own (FG_GEMM_TILE holds for
+# every product): the largest tile, a 160-wide one as stream-K, two stages with
+# K splits, splits that end inside a 16-k stage.
+FORCED = """
+import sys
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests")
+import ferrograd_amd as fg
+import test_gemm_split as t
+t.check_not_finite(fg, "hip", (1000, 785, 601), t.BIG)
+"""
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", ["256,256,32,4,2,1,3", "256,160,32,8,1,0,3", "128,256,32,2,2,2,2", "64,64,8,2,2,3,3"])
+def test_infinities_nan_and_overflow_in_forced_tiles(tile):
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", FORCED, root], env=dict(os.environ, FG_GEMM_TILE=tile), capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+def test_not_finite_products_take_a_few_times_as_long(fg, hip):
+    """A NaN in every tile makes each workgroup compute its tile again on the
+    f32 MFMA, a good half of the split's rate: 2.2 times as long in all, where
+    loads of every element by itself took eleven."""
+    import time
+
+    n = 4096
+    r = np.random.default_rng(8)
+    x, w = (r.standard_normal((n, n)).astype(np.float32) for _ in range(2))
+    bad = x.copy()
+    bad[::16, ::16] = np.nan
+    wt = fg.Tensor.new(w, [n, n], hip)
+    us = []
+    for a in (x, bad):
+        t = fg.Tensor.new(a, [n, n], hip)
+        runs = []
+        for _ in range(5):
+            fg.synchronize(hip)
+            t0 = time.perf_counter()
+            for _ in range(5):
+                t.matmul(wt.permute([1, 0])).realize()
+            fg.synchronize(hip)
+            runs.append(time.perf_counter() - t0)
+        us.append(min(runs))
+    assert us[1] <= 4.0 * us[0], us
