@@ -52,12 +52,15 @@ constexpr uint64_t kZeroBufferTag = 0x5a45524fULL;  // "ZERO"
 // schedule may read its source in place when the copy would not change the
 // layout; a contiguous() the caller asked for is materialised as in the
 // reference.
+constexpr uint64_t kMatmulCopyTag = 0x4d4d4350ULL;  // "MMCP"
 // Int argument of the Sink of a kernel whose output a comparison of the same
 // schedule reads (relu's mask 0 < x): set when fusing. Such a product keeps
 // the f32 MFMA's order of sums and so its bits: a value within rounding of the
 // threshold would otherwise fall on its other side, and with the mask whole
-// terms of the gradient.
+// terms of the gradient. So a product's order depends on what is realised with
+// it: realised before its comparison (a forward pass read before its backward
+// is built) it is split, and the mask follows the split's sums, whose error is
+// no larger.
 constexpr int64_t kComparedSink = 1;
-constexpr uint64_t kMatmulCopyTag = 0x4d4d4350ULL;  // "MMCP"
 
 }  // namespace fg

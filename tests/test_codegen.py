@@ -62,8 +62,13 @@ def test_c3_is_one_mfma_gemm_reading_w_directly(fg, cpu):
     assert [it["class"] for it in items] == ["gemm_mfma_f32"]
     assert len(fg.debug_plan([y], fuse=False)["items"]) == 2  # the copy, then matmul + b
     src = items[0]["source"]
-    assert "__builtin_amdgcn_mfma_f32_32x32x2f32" in src
+    # Nothing compares it: the bfloat16 split, and the f32 MFMA for tiles whose
+    # sums are not finite. Under a relu it is the f32 MFMA's alone.
+    assert "__builtin_amdgcn_mfma_f32_32x32x16_bf16" in src and "__builtin_amdgcn_mfma_f32_32x32x2f32" in src
     compile_only(fg, src, items[0]["name"])
+    under_relu = [it for it in hip_plan(fg, [y, y.relu()]) if it["class"] == "gemm_mfma_f32"]
+    assert len(under_relu) == 1 and "32x32x16_bf16" not in under_relu[0]["source"]
+    assert "__builtin_amdgcn_mfma_f32_32x32x2f32" in under_relu[0]["source"]
 
 
 @pytest.mark.parametrize("mnk,kind", [((256, 128, 784), "small"), ((100, 20, 8192), "small"),

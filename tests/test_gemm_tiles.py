@@ -144,7 +144,8 @@ sys.exit(0 if max(errs.values()) <= 1.0 else 1)
 @pytest.mark.parametrize("tile", ["256,160,16,4,1,3,3", "160,256,32,1,4,2", "256,160,16,4,1,0,3", "128,128,32,2,2,0",
                                   "192,96,32,2,1,2", "96,192,32,1,2,0", "256,256,8,2,2,1", "64,64,24,2,2,1"])
 def test_forced_160_wide_tiles_against_float64(tile):
-    # Tiles the model rarely picks (16-wide k-tiles with three LDS stages; a
+    # Tiles the model rarely picks, on the split products (and below on the f32
+    # MFMA's, whose forms these are: 16-wide k-tiles with three LDS stages; a
     # 160-row tile on every orientation; stream-K, split count 0, with those
     # stages and with two workgroups per CU on ragged 128x128 tiles; waves of
     # three 32-wide tiles, [k][row] stages as a chunk of two and one of one;
@@ -158,6 +159,81 @@ def test_forced_160_wide_tiles_against_float64(tile):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     env = dict(os.environ, FG_GEMM_TILE=tile)
     r = subprocess.run([sys.executable, "-c", FORCED, root], env=env, capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+# The f32 MFMA tiles: products that a comparison of the same schedule reads (a
+# relu's mask). Realised beside its relu, each orientation keeps them; the
+# products above, which nothing compares, are split.
+def compared(fg, p):
+    """The products with their relus, and whether each one's GEMM is split."""
+    split = {}
+    for name, t in p.items():
+        (src,) = [it["source"] for it in fg.debug_plan([t, t.relu()], fuse=True, render_hip=True)["items"]
+                  if it["class"] == "gemm_mfma_f32"]
+        assert "__builtin_amdgcn_mfma_f32_32x32x2f32" in src
+        split[name] = "__builtin_amdgcn_mfma_f32_32x32x16_bf16" in src
+    return [u for t in p.values() for u in (t, t.relu())], split
+
+
+@pytest.mark.parametrize("shape", [(1000, 784, 600), *sorted(CASES)])
+def test_compared_products_keep_the_f32_tiles(fg, cpu, shape):
+    B, fi, fo = shape
+    ones = np.ones
+    p = products(fg, cpu, ones((B, fi), np.float32), ones((fo, fi), np.float32), ones((B, fo), np.float32))
+    assert compared(fg, p)[1] == dict.fromkeys(p, False)
+    for t in p.values():
+        (src,) = [it["source"] for it in fg.debug_plan([t], fuse=True, render_hip=True)["items"]
+                  if it["class"] == "gemm_mfma_f32"]
+        assert "__builtin_amdgcn_mfma_f32_32x32x16_bf16" in src
+
+
+def check_compared(fg, dev, shape):
+    B, fi, fo = shape
+    r = np.random.default_rng(B + fo)
+    x = r.uniform(-1, 1, (B, fi)).astype(np.float32)
+    w = (r.standard_normal((fo, fi)) / np.sqrt(fi)).astype(np.float32)
+    g = r.standard_normal((B, fo)).astype(np.float32)
+    p = products(fg, dev, x, w, g)
+    roots, split = compared(fg, p)
+    assert not any(split.values()), split
+    fg.Tensor.realize_many(roots)
+    x64, w64, g64 = (a.astype(np.float64) for a in (x, w, g))
+    want = {"fwd": (x64 @ w64.T, np.abs(x64) @ np.abs(w64).T), "dx": (g64 @ w64, np.abs(g64) @ np.abs(w64)),
+            "dw": (g64.T @ x64, np.abs(g64).T @ np.abs(x64))}
+    for (name, (v, sc)), t, relu in zip(want.items(), roots[::2], roots[1::2]):
+        got = t.numpy().reshape(v.shape)
+        assert rel_err_bound(got, v, sc, 1e-4) <= 1.0, name
+        assert np.array_equal(relu.numpy().reshape(v.shape), np.maximum(got, 0)), name
+
+
+FORCED_COMPARED = """
+import sys
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests")
+import ferrograd_amd as fg
+import test_gemm_tiles as t
+t.check_compared(fg, "hip", (1000, 784, 600))
+"""
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(520, 608, 300), (601, 617, 333), (3000, 800, 600), (2048, 784, 1000)])
+def test_compared_products_against_float64(fg, hip, shape):
+    check_compared(fg, hip, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", ["256,160,16,4,1,3,3", "160,256,32,1,4,2", "256,160,16,4,1,0,3", "128,128,32,2,2,0",
+                                  "192,96,32,2,1,2", "96,192,32,1,2,0", "256,256,8,2,2,1", "64,64,24,2,2,1"])
+def test_forced_f32_tiles_against_float64(tile):
+    # The forms that the comment of the test above names, on the f32 MFMA.
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", FORCED_COMPARED, root], env=dict(os.environ, FG_GEMM_TILE=tile),
+                       capture_output=True, text=True, timeout=240)
     assert r.returncode == 0, r.stdout + r.stderr
 
 
