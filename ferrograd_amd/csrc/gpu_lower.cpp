@@ -1349,13 +1349,17 @@ bool row_loads_vec4(const UOp& value, const UOp& r_in) {
 // Infinity Cache (10.4 us for the first's 60 MB), below a few MiB by its two
 // launches.
 //
-// From 512 outputs on the unsplit kernel has two workgroups per CU (513 rows
-// of 32,704 run at 6.3 TB/s). Below, the split pays from about 64 steps of an
-// unsplit thread, whose loads then take as long as the second launch: nine
-// rows of 116,508 (114 steps) 8.7 us unsplit, 8.0 us split; rows of 7,281 (28
-// steps) 4.6 us unsplit.
+// The unsplit kernel takes about 0.07 us a step of a thread (0.04 from the
+// caches, 0.09 where 64 workgroups read 67 MB) and reads 7.2 TB/s from 256
+// outputs on; the split 6.5 TB/s and a second launch, which costs the host 4 us
+// (a call with one launch takes 6.8 us, with two 10.5). So it is taken where
+// the estimate is 2 us better: 64 rows of 2^18 terms 23.6 -> 12.6 us of
+// kernels, 100 rows of 100,001 a call of 32 -> 11 us; not for one row of 65,536
+// (6.8 us a call, 10.9 split), 300 of 20,001 (7.4, 10.9), 500 of 65,536 (18.1,
+// 20.5) or 256 of 2^18 (36.8, 40.4).
 constexpr int64_t kRowSplitMaxOutputs = 512;
-constexpr int64_t kRowSplitMinSteps = 64;
+constexpr double kRowSplitStepUs = 0.07, kRowReadBytesPerUs = 7.2e6, kRowSplitReadBytesPerUs = 6.5e6;
+constexpr double kRowSplitSecondLaunchUs = 4.0, kRowSplitCallUs = 10.5, kRowSplitGainUs = 2.0;
 constexpr int64_t kRowSplitWorkgroups = 2048;  // eight 256-thread workgroups per CU
 constexpr int64_t kRowSplitChunkSteps = 8;     // fewest steps of a chunk's threads
 
@@ -1371,10 +1375,18 @@ struct RowSplit {
 // `steps`: the steps a thread of the unsplit kernel runs.
 bool row_split(const KernelInfo& ki, const RowTerms& rt, int64_t steps, RowSplit* sp) {
   const int64_t nout = total_outputs(ki);
-  if (nout >= kRowSplitMaxOutputs || steps < kRowSplitMinSteps) return false;
-  if (rt.terms >= (int64_t(1) << 31) - (int64_t(1) << 20)) return false;
-  for (auto& ld : loads_in(rt.value))
-    if (!affine_of(ld.src(0).src(1)).ok) return false;
+  if (nout >= kRowSplitMaxOutputs || rt.terms >= (int64_t(1) << 31) - (int64_t(1) << 20)) return false;
+  double bytes = 0.0;  // read by all outputs
+  for (auto& ld : loads_in(rt.value)) {
+    const Affine a = affine_of(ld.src(0).src(1));
+    if (!a.ok) return false;
+    bool own = false;
+    for (auto& r : ki.out_ranges) own = own || a.coef(r) != 0;
+    bytes += 4.0 * static_cast<double>(rt.terms) * static_cast<double>(own ? nout : 1);
+  }
+  const double whole_us = 1.0 + std::max(kRowSplitStepUs * static_cast<double>(steps), bytes / kRowReadBytesPerUs);
+  const double split_us = std::max(kRowSplitCallUs, bytes / kRowSplitReadBytesPerUs + kRowSplitSecondLaunchUs);
+  if (whole_us < split_us + kRowSplitGainUs) return false;
   sp->value = rt.value;
   sp->ranges = rt.ranges;
   const int64_t L = range_extent(rt.ranges.back());

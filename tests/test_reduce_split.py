@@ -56,3 +56,12 @@ def test_split_row_reduction_launches(fg, cpu):
     # An empty reduction keeps its one pass and its identity.
     e = fg.Tensor.zeros([0, 3], cpu).sum([0, 1])
     assert "_part(" not in fg.debug_plan([e], fuse=True, render_hip=True)["items"][0]["source"]
+
+
+@pytest.mark.parametrize("shape,split", [((1, 65536), False), ((1, 1 << 20), True), ((3, 70000), False), ((64, 1 << 18), True),
+                                         ((300, 20001), False), ((100, 100001), True), ((500, 65536), False), ((256, 1 << 18), False),
+                                         ((511, 40000), False)])
+def test_rows_are_split_where_a_second_launch_pays(fg, cpu, shape, split):
+    x = fg.Tensor.zeros(list(shape), cpu).add(fg.Tensor.scalar(1.0, cpu)).realize()
+    (item,) = fg.debug_plan([x.mul(x).sum([1])], fuse=True, render_hip=True)["items"]
+    assert item["class"] == "row_reduce" and ("_part(" in item["source"]) == split
