@@ -2852,6 +2852,135 @@ int64_t stream_k_tile_period(int64_t ntiles, int64_t kt, int64_t G) {
   return 0;
 }
 
+// The end of either tiled GEMM, behind the store loop's `if (grow < M_ && gcol <
+// N_) {`: the epilogue, or the partial sums of a split and the pass that adds
+// them; then the launches.
+RenderedKernel finish_gemm(const KernelInfo& ki, const GemmMatch& g, const std::string& name, const GemmTile& tile, int64_t sk_D,
+                           const std::function<std::string(const std::string&, int, bool)>& sig, std::ostringstream& s,
+                           bool f32_tiles) {
+  const int64_t M = g.M, N = g.N, S = tile.S, NP = (N + 3) / 4 * 4;
+  const bool split = S > 1 || tile.stream_k;
+  auto indent = [](const std::string& code, const std::string& pre) {
+    std::ostringstream o;
+    std::istringstream is(code);
+    std::string l;
+    while (std::getline(is, l)) o << pre << l << "\n";
+    return o.str();
+  };
+  // Everything outside the reduction, for the four columns gcol..gcol+3 of
+  // row grow whose sums are in gv.
+  auto epilogue = [&]() {
+    static const char* kComp[4] = {"gv.x", "gv.y", "gv.z", "gv.w"};
+    Emitter em;
+    em.define_range(g.rm, "grow");
+    const std::string out = pname(ki.out_param);
+    if (N % 4 == 0) {
+      // Every column group lies inside the tile: lanes along the columns.
+      em.define_range(g.rn, "gcol");
+      em.set_lane_range(g.rn, 4);
+      em.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
+        FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
+        return kComp[lane];
+      };
+      std::vector<std::string> vals;
+      for (int u = 0; u < 4; u++) vals.push_back(em.val(ki.value, u));
+      Affine ao = affine_of(ki.out_index);
+      bool vstore = ao.ok && ao.coef(g.rn) == 1 && ao.c0 % 4 == 0 &&
+                    ki.out_param.dtype().kind == DTypeKind::F32;
+      for (auto& t : ao.terms)
+        if (t.first != g.rn && t.second % 4 != 0) vstore = false;
+      if (vstore) {
+        em.line("*(float4*)(" + out + "+" + em.idx(ki.out_index, 0) + ") = make_float4(" + vals[0] + ", " + vals[1] +
+                ", " + vals[2] + ", " + vals[3] + ");");
+      } else {
+        for (int u = 0; u < 4; u++) em.line(out + "[" + em.idx(ki.out_index, u) + "] = " + vals[u] + ";");
+      }
+    } else {
+      // Ragged last column group: one guarded column at a time.
+      for (int u = 0; u < 4; u++) {
+        const std::string col = "(gcol+" + std::to_string(u) + ")";
+        em.open_scope("if (" + col + " < N_) {", "}");
+        em.define_range(g.rn, col);
+        em.reduce_cb_ = [&, u](const UOp& RR, int) -> std::string {
+          FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
+          return kComp[u];
+        };
+        std::string v = em.val(ki.value, 0);
+        em.line(out + "[" + em.idx(ki.out_index, 0) + "] = " + v + ";");
+        em.close_scope();
+      }
+    }
+    return em.code();
+  };
+  if (!split) {
+    s << indent(epilogue(), "        ");
+  } else {
+    // Raw partial sums of this K range; the epilogue runs after they are summed.
+    s << "        *(fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol) = gv;\n";
+  }
+  s << "      }\n    }\n    __syncthreads();\n  }\n";
+  if (tile.stream_k) s << "  }\n";  // the workgroup's next segment
+  s << "}\n";
+  if (split) {
+    // Second pass: one thread per 4 columns of a row sums the partials in
+    // split order (stream-K: the tile's segments, in k order), then runs the
+    // epilogue.
+    s << sig(name + "_fin", 256, false) << " {\n";
+    s << R"(  const long gid = (long)blockIdx.x * 256 + threadIdx.x;
+  if (gid >= (long)M_ * (NP_ / 4)) return;
+  const int grow = (int)(gid / (NP_ / 4)), gcol = (int)(gid % (NP_ / 4)) * 4;
+  fg_f4 gv = *(const fg_f4*)(fg_scratch + (long)grow * NP_ + gcol);
+)";
+    if (tile.stream_k && sk_D > 0) {
+      // The tile's block index (the inverse of the main pass's row-major
+      // slot), then how many workgroups its k-tiles were split over.
+      s << R"(  const int nbn = (N_ + BN - 1) / BN, sq = (grow / BM) * nbn + gcol / BN;
+  const long t0 = (long)((sq % (NTILES_ / SK_D_)) * SK_D_ + sq / (NTILES_ / SK_D_)) * KTT_;
+  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
+  for (int ks = 1; ks < nseg; ks++) {)";
+    } else if (tile.stream_k) {
+      // The tile's block index (the inverse of the main pass's grouped
+      // order), then how many workgroups its k-tiles were split over.
+      s << R"(  const int nbm = (M_ + BM - 1) / BM, nbn = (N_ + BN - 1) / BN, GM = 8;
+  const int tm = grow / BM, tn = gcol / BN, group = tm / GM, first_m = group * GM;
+  const int gsz = (nbm - first_m) < GM ? (nbm - first_m) : GM;
+  const long t0 = (long)(group * GM * nbn + tn * gsz + (tm - first_m)) * KTT_;
+  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
+  for (int ks = 1; ks < nseg; ks++) {)";
+    } else {
+      s << "  for (int ks = 1; ks < S_; ks++) {";
+    }
+    s << R"(
+    const fg_f4 p = *(const fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol);
+    gv.x = gv.x + p.x; gv.y = gv.y + p.y; gv.z = gv.z + p.z; gv.w = gv.w + p.w;
+  }
+  if (gcol < N_) {
+)";
+    s << indent(epilogue(), "    ");
+    s << "  }\n}\n";
+  }
+  RenderedKernel rk;
+  rk.name = name;
+  rk.kind = kernel_class_name(KernelClass::Gemm);
+  rk.source = s.str();
+  if (f32_tiles && tile.nbuf == 3) rk.source = gemm_three_stages(rk.source);
+  rk.block[0] = static_cast<unsigned>(tile.nt());
+  rk.grid[0] = static_cast<unsigned>(tile.stream_k ? tile.G : (M + tile.BM - 1) / tile.BM * ((N + tile.BN - 1) / tile.BN) * S);
+  if (tile.stream_k) rk.source = gemm_stream_k(rk.source, sk_D);
+  if (split) {
+    LaunchSpec a, b;
+    a.func = name + "_part";
+    a.grid[0] = rk.grid[0];
+    a.block[0] = static_cast<unsigned>(tile.nt());
+    b.func = name + "_fin";
+    b.grid[0] = static_cast<unsigned>((M * (NP / 4) + 255) / 256);
+    b.block[0] = 256;
+    rk.launches = {a, b};
+    rk.scratch_bytes = static_cast<size_t>(S * M * NP) * sizeof(float);
+  }
+  return rk;
+}
+
 // ── Tiled GEMM on the f32 MFMA ──────────────────────────────────────────────
 // For two kinds of products; the others run on the split tiles below.
 // - Products a comparison of the same schedule reads (KernelInfo::compared, a
@@ -3258,125 +3387,7 @@ RenderedKernel render_gemm_f32(const KernelInfo& ki, const GemmMatch& g, const s
       const int gcol = n0 + wn + cc;
       if (grow < M_ && gcol < N_) {
 )";
-  // Everything outside the reduction, for the four columns gcol..gcol+3 of
-  // row grow whose sums are in gv.
-  auto epilogue = [&]() {
-    static const char* kComp[4] = {"gv.x", "gv.y", "gv.z", "gv.w"};
-    Emitter em;
-    em.define_range(g.rm, "grow");
-    const std::string out = pname(ki.out_param);
-    if (N % 4 == 0) {
-      // Every column group lies inside the tile: lanes along the columns.
-      em.define_range(g.rn, "gcol");
-      em.set_lane_range(g.rn, 4);
-      em.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
-        FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
-        return kComp[lane];
-      };
-      std::vector<std::string> vals;
-      for (int u = 0; u < 4; u++) vals.push_back(em.val(ki.value, u));
-      Affine ao = affine_of(ki.out_index);
-      bool vstore = ao.ok && ao.coef(g.rn) == 1 && ao.c0 % 4 == 0 &&
-                    ki.out_param.dtype().kind == DTypeKind::F32;
-      for (auto& t : ao.terms)
-        if (t.first != g.rn && t.second % 4 != 0) vstore = false;
-      if (vstore) {
-        em.line("*(float4*)(" + out + "+" + em.idx(ki.out_index, 0) + ") = make_float4(" + vals[0] + ", " + vals[1] +
-                ", " + vals[2] + ", " + vals[3] + ");");
-      } else {
-        for (int u = 0; u < 4; u++) em.line(out + "[" + em.idx(ki.out_index, u) + "] = " + vals[u] + ";");
-      }
-    } else {
-      // Ragged last column group: one guarded column at a time.
-      for (int u = 0; u < 4; u++) {
-        const std::string col = "(gcol+" + std::to_string(u) + ")";
-        em.open_scope("if (" + col + " < N_) {", "}");
-        em.define_range(g.rn, col);
-        em.reduce_cb_ = [&, u](const UOp& RR, int) -> std::string {
-          FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
-          return kComp[u];
-        };
-        std::string v = em.val(ki.value, 0);
-        em.line(out + "[" + em.idx(ki.out_index, 0) + "] = " + v + ";");
-        em.close_scope();
-      }
-    }
-    return em.code();
-  };
-  auto indent = [](const std::string& code, const std::string& pre) {
-    std::ostringstream o;
-    std::istringstream is(code);
-    std::string l;
-    while (std::getline(is, l)) o << pre << l << "\n";
-    return o.str();
-  };
-  if (!split) {
-    s << indent(epilogue(), "        ");
-  } else {
-    // Raw partial sums of this K range; the epilogue runs after they are summed.
-    s << "        *(fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol) = gv;\n";
-  }
-  s << "      }\n    }\n    __syncthreads();\n  }\n";
-  if (tile.stream_k) s << "  }\n";  // the workgroup's next segment
-  s << "}\n";
-  if (split) {
-    // Second pass: one thread per 4 columns of a row sums the partials in
-    // split order (stream-K: the tile's segments, in k order), then runs the
-    // epilogue.
-    s << sig(name + "_fin", 256, false) << " {\n";
-    s << R"(  const long gid = (long)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= (long)M_ * (NP_ / 4)) return;
-  const int grow = (int)(gid / (NP_ / 4)), gcol = (int)(gid % (NP_ / 4)) * 4;
-  fg_f4 gv = *(const fg_f4*)(fg_scratch + (long)grow * NP_ + gcol);
-)";
-    if (tile.stream_k && sk_D > 0) {
-      // The tile's block index (the inverse of the main pass's row-major
-      // slot), then how many workgroups its k-tiles were split over.
-      s << R"(  const int nbn = (N_ + BN - 1) / BN, sq = (grow / BM) * nbn + gcol / BN;
-  const long t0 = (long)((sq % (NTILES_ / SK_D_)) * SK_D_ + sq / (NTILES_ / SK_D_)) * KTT_;
-  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
-  for (int ks = 1; ks < nseg; ks++) {)";
-    } else if (tile.stream_k) {
-      // The tile's block index (the inverse of the main pass's grouped
-      // order), then how many workgroups its k-tiles were split over.
-      s << R"(  const int nbm = (M_ + BM - 1) / BM, nbn = (N_ + BN - 1) / BN, GM = 8;
-  const int tm = grow / BM, tn = gcol / BN, group = tm / GM, first_m = group * GM;
-  const int gsz = (nbm - first_m) < GM ? (nbm - first_m) : GM;
-  const long t0 = (long)(group * GM * nbn + tn * gsz + (tm - first_m)) * KTT_;
-  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
-  for (int ks = 1; ks < nseg; ks++) {)";
-    } else {
-      s << "  for (int ks = 1; ks < S_; ks++) {";
-    }
-    s << R"(
-    const fg_f4 p = *(const fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol);
-    gv.x = gv.x + p.x; gv.y = gv.y + p.y; gv.z = gv.z + p.z; gv.w = gv.w + p.w;
-  }
-  if (gcol < N_) {
-)";
-    s << indent(epilogue(), "    ");
-    s << "  }\n}\n";
-  }
-  RenderedKernel rk;
-  rk.name = name;
-  rk.kind = kernel_class_name(KernelClass::Gemm);
-  rk.source = s.str();
-  if (tile.nbuf == 3) rk.source = gemm_three_stages(rk.source);
-  rk.block[0] = static_cast<unsigned>(NT);
-  rk.grid[0] = static_cast<unsigned>(tile.stream_k ? tile.G : ntiles * S);
-  if (tile.stream_k) rk.source = gemm_stream_k(rk.source, sk_D);
-  if (split) {
-    LaunchSpec a, b;
-    a.func = name + "_part";
-    a.grid[0] = rk.grid[0];
-    a.block[0] = static_cast<unsigned>(NT);
-    b.func = name + "_fin";
-    b.grid[0] = static_cast<unsigned>((M * (NP / 4) + 255) / 256);
-    b.block[0] = 256;
-    rk.launches = {a, b};
-    rk.scratch_bytes = static_cast<size_t>(S * M * NP) * sizeof(float);
-  }
-  return rk;
+  return finish_gemm(ki, g, name, tile, sk_D, sig, s, true);
 }
 
 // ── Tiled GEMM on the bfloat16 matrix cores, at f32 precision ──────────────
@@ -3840,117 +3851,7 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
       const int grow = m0 + wm + 32 * i + rr, gcol = n0 + wn + EW * jj + cc;
       if (grow < M_ && gcol < N_) {
 )";
-  // Everything outside the reduction, for the four columns gcol..gcol+3 of
-  // row grow whose sums are in gv.
-  auto epilogue = [&]() {
-    static const char* kComp[4] = {"gv.x", "gv.y", "gv.z", "gv.w"};
-    Emitter em;
-    em.define_range(g.rm, "grow");
-    const std::string out = pname(ki.out_param);
-    if (N % 4 == 0) {
-      // Every column group lies inside the tile: lanes along the columns.
-      em.define_range(g.rn, "gcol");
-      em.set_lane_range(g.rn, 4);
-      em.reduce_cb_ = [&](const UOp& RR, int lane) -> std::string {
-        FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
-        return kComp[lane];
-      };
-      std::vector<std::string> vals;
-      for (int u = 0; u < 4; u++) vals.push_back(em.val(ki.value, u));
-      Affine ao = affine_of(ki.out_index);
-      bool vstore = ao.ok && ao.coef(g.rn) == 1 && ao.c0 % 4 == 0 &&
-                    ki.out_param.dtype().kind == DTypeKind::F32;
-      for (auto& t : ao.terms)
-        if (t.first != g.rn && t.second % 4 != 0) vstore = false;
-      if (vstore) {
-        em.line("*(float4*)(" + out + "+" + em.idx(ki.out_index, 0) + ") = make_float4(" + vals[0] + ", " + vals[1] +
-                ", " + vals[2] + ", " + vals[3] + ");");
-      } else {
-        for (int u = 0; u < 4; u++) em.line(out + "[" + em.idx(ki.out_index, u) + "] = " + vals[u] + ";");
-      }
-    } else {
-      // Ragged last column group: one guarded column at a time.
-      for (int u = 0; u < 4; u++) {
-        const std::string col = "(gcol+" + std::to_string(u) + ")";
-        em.open_scope("if (" + col + " < N_) {", "}");
-        em.define_range(g.rn, col);
-        em.reduce_cb_ = [&, u](const UOp& RR, int) -> std::string {
-          FG_CHECK(RR == g.R, "gemm epilogue sees one reduction");
-          return kComp[u];
-        };
-        std::string v = em.val(ki.value, 0);
-        em.line(out + "[" + em.idx(ki.out_index, 0) + "] = " + v + ";");
-        em.close_scope();
-      }
-    }
-    return em.code();
-  };
-  if (!split) {
-    s << indent(epilogue(), "        ");
-  } else {
-    // Raw partial sums of this K range; the epilogue runs after they are summed.
-    s << "        *(fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol) = gv;\n";
-  }
-  s << "      }\n    }\n    __syncthreads();\n  }\n";
-  if (tile.stream_k) s << "  }\n";  // the workgroup's next segment
-  s << "}\n";
-  if (split) {
-    // Second pass: one thread per 4 columns of a row sums the partials in
-    // split order (stream-K: the tile's segments, in k order), then runs the
-    // epilogue.
-    s << sig(name + "_fin", 256, false) << " {\n";
-    s << R"(  const long gid = (long)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= (long)M_ * (NP_ / 4)) return;
-  const int grow = (int)(gid / (NP_ / 4)), gcol = (int)(gid % (NP_ / 4)) * 4;
-  fg_f4 gv = *(const fg_f4*)(fg_scratch + (long)grow * NP_ + gcol);
-)";
-    if (tile.stream_k && sk_D > 0) {
-      // The tile's block index (the inverse of the main pass's row-major
-      // slot), then how many workgroups its k-tiles were split over.
-      s << R"(  const int nbn = (N_ + BN - 1) / BN, sq = (grow / BM) * nbn + gcol / BN;
-  const long t0 = (long)((sq % (NTILES_ / SK_D_)) * SK_D_ + sq / (NTILES_ / SK_D_)) * KTT_;
-  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
-  for (int ks = 1; ks < nseg; ks++) {)";
-    } else if (tile.stream_k) {
-      // The tile's block index (the inverse of the main pass's grouped
-      // order), then how many workgroups its k-tiles were split over.
-      s << R"(  const int nbm = (M_ + BM - 1) / BM, nbn = (N_ + BN - 1) / BN, GM = 8;
-  const int tm = grow / BM, tn = gcol / BN, group = tm / GM, first_m = group * GM;
-  const int gsz = (nbm - first_m) < GM ? (nbm - first_m) : GM;
-  const long t0 = (long)(group * GM * nbn + tn * gsz + (tm - first_m)) * KTT_;
-  const int nseg = fg_sk_owner(t0 + KTT_ - 1) - fg_sk_owner(t0) + 1;
-  for (int ks = 1; ks < nseg; ks++) {)";
-    } else {
-      s << "  for (int ks = 1; ks < S_; ks++) {";
-    }
-    s << R"(
-    const fg_f4 p = *(const fg_f4*)(fg_scratch + ((long)ks * M_ + grow) * NP_ + gcol);
-    gv.x = gv.x + p.x; gv.y = gv.y + p.y; gv.z = gv.z + p.z; gv.w = gv.w + p.w;
-  }
-  if (gcol < N_) {
-)";
-    s << indent(epilogue(), "    ");
-    s << "  }\n}\n";
-  }
-  RenderedKernel rk;
-  rk.name = name;
-  rk.kind = kernel_class_name(KernelClass::Gemm);
-  rk.source = s.str();
-  rk.block[0] = static_cast<unsigned>(NT);
-  rk.grid[0] = static_cast<unsigned>(tile.stream_k ? tile.G : ntiles * S);
-  if (tile.stream_k) rk.source = gemm_stream_k(rk.source, sk_D);
-  if (split) {
-    LaunchSpec a, b;
-    a.func = name + "_part";
-    a.grid[0] = rk.grid[0];
-    a.block[0] = static_cast<unsigned>(NT);
-    b.func = name + "_fin";
-    b.grid[0] = static_cast<unsigned>((M * (NP / 4) + 255) / 256);
-    b.block[0] = 256;
-    rk.launches = {a, b};
-    rk.scratch_bytes = static_cast<size_t>(S * M * NP) * sizeof(float);
-  }
-  return rk;
+  return finish_gemm(ki, g, name, tile, sk_D, sig, s, false);
 }
 
 // ── Block: a small kernel in one workgroup ──────────────────────────────────
