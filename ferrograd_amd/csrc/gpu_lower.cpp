@@ -2138,10 +2138,12 @@ std::vector<KmChunk> km_chunks(int T) {
 }
 
 constexpr int kGemmStageK = 16;         // k of one LDS stage of the tiled GEMM, one MFMA deep
-// Stages whose products are summed apart (see render_gemm): every one up to K
-// kGemmFoldAllK; every 2nd up to kGemmFold2K and for waves of at most
-// kGemmFoldTiles tiles of 32x32; else every 4th.
-constexpr int64_t kGemmFoldAllK = 1024, kGemmFold2K = 2048;
+// Stages whose products are summed apart (see render_gemm): every 2nd for waves
+// of at most kGemmFoldTiles tiles of 32x32, else every 4th; every one up to K
+// kGemmFoldAllK where the f32 tiles would run shorter chains of sums. With chains
+// of one length every 2nd gives two thirds of the f32 tiles' error (3000x1500 of
+// K 128 1.3e-7 and 2.0e-7), so for it shorter means two thirds or less.
+constexpr int64_t kGemmFoldAllK = 1024;
 constexpr int kGemmFoldTiles = 5;
 constexpr int64_t kLdsPerCu = 163840;   // gfx950 LDS bytes per CU
 constexpr int64_t kMinSplitK = 64;      // shortest K range a split workgroup runs
@@ -3407,13 +3409,13 @@ RenderedKernel render_gemm_f32(const KernelInfo& ki, const GemmMatch& g, const s
 //
 // Error against 64 bits (2-norm): the six products are added to the running
 // sums one after another, smallest first, except in the stages whose products
-// are summed apart and added once: every 4th, every 2nd for waves of few tiles
-// and up to a K of 2048, and every one up to 1024, where the f32 tiles keep
-// their chains short by splitting K. With every 2nd, 1030x1010 of K 320 had an
-// error of 2.06e-7 (positive operands 1.62e-7), now 9.9e-8 (6.9e-8); the f32
-// tiles 1.51e-7 (6.7e-8). It costs 0-5% there (4096x1024 of K 784 53.1 -> 55.3
-// us), 25% at 3000x1500 of K 1500. Of 50 products of 33 to 4096 k none is above
-// the f32 tiles, of positive operands a few (by up to 9%). The
+// are summed apart and added once: every 4th, every 2nd for waves of few tiles,
+// and every one up to a K of 1024 where the f32 tiles would keep their chains
+// shorter by splitting K. With every 2nd, 1030x1010 of K 320 had an error of
+// 2.06e-7 (positive operands 1.62e-7), now 9.9e-8 (6.9e-8); the f32 tiles
+// 1.51e-7 (6.7e-8). It costs 0-7% there (4096x1024 of K 784 53.1 -> 55.3 us),
+// 25% at 3000x1500 of K 1500. Of 50 products of 33 to 4096 k none is above the
+// f32 tiles, of positive operands a few (by up to 9%). The
 // bfloat16 MFMA rounds the aligned sum down, so the operands' odd rows are
 // negated and the results' signs alternate: without that the errors of all
 // sums leaned the same way (mean -2.1e-7 of their spread at K 4096, 1e-10
@@ -3485,7 +3487,16 @@ RenderedKernel render_gemm(const KernelInfo& ki, const GemmMatch& g, const std::
   s << "#define S_ " << S << "\n#define KC_ " << KC << "\n#define NTILES_ " << ntiles << "\n";
   s << "#define BM " << BM << "\n#define BN " << BN << "\n#define BK " << BK << "\n";
   s << "#define NT " << NT << "\n#define WGN " << WGN << "\n#define TM " << TM << "\n#define TN " << TN << "\n";
-  s << "#define NBUF_ " << tile.nbuf << "\n#define FOLD_ " << (K <= kGemmFoldAllK ? 1 : K <= kGemmFold2K || TM * TN <= kGemmFoldTiles ? 2 : 4) << "\n";
+  // The k that one running sum goes through.
+  auto chain = [&](const GemmTile& t) {
+    const int64_t nt = ((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN), kt = (K + t.BK - 1) / t.BK;
+    return std::min(K, t.stream_k ? (nt * kt + t.G - 1) / t.G * t.BK : t.KC);
+  };
+  GemmTile forced;
+  const bool fold_2nd = TM * TN <= kGemmFoldTiles;
+  const int64_t f32_chain = K <= kGemmFoldAllK && !gemm_tile_override(&forced) ? chain(choose_gemm_tile_f32(M, N, K)) : K;
+  const bool fold_all = fold_2nd ? 3 * f32_chain <= 2 * chain(tile) : f32_chain < chain(tile);
+  s << "#define NBUF_ " << tile.nbuf << "\n#define FOLD_ " << (fold_all ? 1 : fold_2nd ? 2 : 4) << "\n";
   if (tile.stream_k) {
     s << "#define G_ " << tile.G << "\n#define KTT_ " << KTT << "\n#define ITERS_ " << ntiles * KTT << "L\n";
     if (sk_D > 0) s << "#define SK_D_ " << sk_D << "\n";
